@@ -465,8 +465,29 @@ bool is_1d1d(const Operands& o, const Recipe& r) {
            r.gran_k_b == 128;
 }
 
-// The 1D1D kernels: the 128 x 128 LDS-pipelined one (variant 7, the default) or
-// the 128-row streaming one (variant 6, by tile override).
+// Tile of the pipelined 1D1D kernel. 256 x 256 (one workgroup per CU) moves half of
+// the 128 x 128 tile's bytes from L2 to LDS per FLOP; 128 x 128 (two per CU) runs
+// one workgroup's FP32 C / D epilogue under the other's K loop and fills part-empty
+// rounds better. Time per round of resident tiles, measured (us, kb = K blocks of a
+// tile): 128 x 128 10.4 + 1.41 kb, 256 x 256 20.8 + 2.32 kb for twice the outputs,
+// and a part-empty round costs about half of what it leaves empty. Measured, 128 ->
+// 256: 8 groups 4096 x 7168, kb 32 1582-1596 -> 1353-1360, 8 x 7168 x 4096 at kb 8
+// 607 -> 550; 4096 x 4096 at kb 32 108 -> 96, at kb 8 44 -> 45; 7168 x 2048 at kb 32
+// (224 tiles of 256) 104 -> 106, 8 x 576 x 4096 at kb 16 88 -> 100.
+// kb: the mean over the groups (k: the sum of their K).
+TileConfig choose_tile_1d1d(int64_t m, int64_t n, int64_t k, int64_t groups, int cus) {
+    const double kb = (double)k / 128 / (double)std::max<int64_t>(groups, 1);
+    auto rounds = [&](int64_t tile, int64_t slots) {
+        const int64_t tiles = ceil_div(m, tile) * ceil_div(n, tile) * groups;
+        return std::max(1.0, 0.5 * ((double)ceil_div(tiles, slots) + (double)tiles / (double)slots));
+    };
+    const double c128 = rounds(128, 2 * (int64_t)cus) * (10.4 + 1.41 * kb);
+    const double c256 = 8.0 + rounds(256, cus) * (20.8 + 2.32 * kb);
+    return c256 < 0.97 * c128 ? TileConfig{256, 256, 7} : TileConfig{128, 128, 7};
+}
+
+// The 1D1D kernels: the LDS-pipelined one (variant 7, the default) or the 128-row
+// streaming one (variant 6, by tile override).
 void launch_1d1d(bool k_grouped, const Fp8GemmArgs& args, hipStream_t stream, int64_t m, int64_t n, int64_t k,
                  int64_t groups) {
     const GemmKind kind = k_grouped ? kKGrouped : kNormal;
@@ -476,8 +497,12 @@ void launch_1d1d(bool k_grouped, const Fp8GemmArgs& args, hipStream_t stream, in
         launch_fp8_gemm_1d1d(k_grouped, waves, args, stream);
         return;
     }
-    record_config("fp8_gemm_1d1d", kind, TileConfig{128, 128, 7}, m, n, k, groups);
-    launch_fp8_gemm_1d1d_pipe(k_grouped, args, stream);
+    int cus = 256;
+    try { cus = num_sms_now(); } catch (const Error&) {}
+    TileConfig t = choose_tile_1d1d(m, n, k, groups, std::max(1, cus));
+    if (g_tile_variant.load() == 7) t.block_m = g_tile_m.load(), t.block_n = g_tile_n.load();
+    record_config("fp8_gemm_1d1d", kind, t, m, n, k, groups);
+    launch_fp8_gemm_1d1d_pipe(k_grouped, t, args, stream);
 }
 
 bool is_ue8m0_path(const Operands& o, const Recipe& r) {
@@ -1675,7 +1700,7 @@ int dg_set_tile_override(int32_t variant, int32_t block_m, int32_t block_n) {
                                           block_n % 32 == 0 && block_n >= 128 &&
                                           block_n <= 256)
                         : variant == 6 ? (block_m == 128 && (block_n == 128 || block_n == 192 || block_n == 256))
-                        : variant == 7 ? (block_m == 128 && block_n == 128)
+                        : variant == 7 ? (block_m == block_n && (block_m == 128 || block_m == 256))
                         : variant == 8 || variant == 9
                             ? ((block_m == 16 || block_m == 32 || block_m == kTinyMRows) &&
                                (block_n == 16 || block_n == 32 || block_n == 64))

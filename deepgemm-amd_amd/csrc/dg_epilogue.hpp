@@ -44,9 +44,10 @@ struct RowEpilogue {
     static_assert(WN % VPL == 0 && LPR <= 64, "row split");
 
     // Rows staged per pass for a region of `bytes` (a multiple of 32, at most WM).
+    // With C, passes of 32 rows: the next pass's C is loaded while one is stored.
     static constexpr int rows_per_pass(int bytes) {
         const int r = bytes / ROW_BYTES / 32 * 32;
-        return r > WM ? WM : r;
+        return HAS_C ? 32 : r > WM ? WM : r;
     }
 
     // 16-byte unit u of staged row r: XOR swizzle when a row has a power-of-two
@@ -89,10 +90,14 @@ struct RowEpilogue {
         }
         // ---- C, loaded ahead of the stores: a load placed after a store would
         // wait for it (C may be D itself, so the compiler keeps them in order),
-        // one memory round trip per row segment. So each pass loads all of its C
-        // once its accumulators are staged, before its stores. (Loading the next
-        // pass's C there too spills registers.) Every element is still read
-        // before it is written. Only whole VPL-wide
+        // one memory round trip per row segment. So the first pass's C is loaded
+        // before its accumulators are staged, and each later pass's C before the
+        // stores of the one before it: with 32-row passes that is two passes of C
+        // in registers, and a pass's loads arrive while the last one is staged
+        // and stored. (With 64-row
+        // passes, each loading its own C: K-grouped, 128 x 128 tiles, 1640-1650
+        // against 1590-1605 us; FP32 C, 4096 x 4096 x 7168, 121.5 against 119.5.)
+        // Every element is still read before it is written. Only whole VPL-wide
         // segments of stored rows are prefetched, and nothing else is written to
         // cpre (a merged default value would make the compiler copy, and so wait
         // for, each load right away); the rare partial segment at the right edge
@@ -124,6 +129,7 @@ struct RowEpilogue {
                 }
             }
         };
+        if constexpr (HAS_C) prefetch_c(0);
 #pragma unroll
         for (int p0 = 0; p0 < WM; p0 += RPP) {
             // ---- registers -> LDS (rows p0 .. p0 + RPP of the wave tile)
@@ -146,7 +152,8 @@ struct RowEpilogue {
                         }
                     }
             }
-            if constexpr (HAS_C) prefetch_c(p0 / RPP);
+            if constexpr (HAS_C)
+                if (p0 + RPP < WM) prefetch_c(p0 / RPP + 1);
             if constexpr (!std::is_same_v<std::decay_t<Hook>, NoEpilogueHook>) {
                 // After the first pass is staged (the row flags' index loads return
                 // meanwhile) and before anything is read back. The flags stay ahead of

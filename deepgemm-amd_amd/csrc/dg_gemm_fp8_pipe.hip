@@ -57,6 +57,28 @@ constexpr int kMaxKBlocksKsa = 256;
 
 __device__ __forceinline__ int swz_g(int r) { return ((r >> 1) ^ ((r & 1) << 2)) & 7; }
 
+// Lane E of each row of 16 lanes, given to the whole row (DPP row_newbcast). As a
+// multiply's operand it folds into v_mul_f32_dpp: no register and no instruction
+// of its own.
+template <int E>
+__device__ __forceinline__ float row_lane(float v) {
+    static_assert(E >= 0 && E < 16, "lane of a 16-lane row");
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + E, 0xf, 0xf, true));
+}
+// fin[E ..] = fma(sa * sb[e], acc[e], fin[e]) for four elements, sb[e] in lane e of
+// the lane's row of 16. The four multiplies come first: a DPP instruction may not
+// write a register that one of the two instructions before it wrote, and one
+// temporary for all would put an s_nop between every two of them.
+template <int E>
+__device__ __forceinline__ void promote_bcast4(f32x16& fin, const f32x16& acc, float sa, float sb) {
+    const float p0 = sa * row_lane<E>(sb), p1 = sa * row_lane<E + 1>(sb);
+    const float p2 = sa * row_lane<E + 2>(sb), p3 = sa * row_lane<E + 3>(sb);
+    fin[E] = __builtin_fmaf(p0, acc[E], fin[E]);
+    fin[E + 1] = __builtin_fmaf(p1, acc[E + 1], fin[E + 1]);
+    fin[E + 2] = __builtin_fmaf(p2, acc[E + 2], fin[E + 2]);
+    fin[E + 3] = __builtin_fmaf(p3, acc[E + 3], fin[E + 3]);
+}
+
 // KT: K is not a multiple of 128 (the last K block is partial).
 // PERSIST: persistent workgroups (grid = CU count) walk the launch's tile
 // sequence with stride gridDim.x, the reference's scheduler
@@ -322,6 +344,8 @@ fp8_gemm_1d2d_pipe_kernel(const Fp8GemmArgs p_arg, const int num_m_blocks, const
     const int sa_row = wave * SA_ROWS_PER_WAVE + lane;
     const uint32_t voff_sa = (uint32_t)(min(sa_row, a_rows - 1) * p.sfa_sm) * 4u;
     const int sb_seg = min(wave, SB_SEGS - 1);   // SB1D: surplus waves repeat the last segment
+    // SB1D: the column (of 32) whose scale this lane holds
+    const int sb_lane = ((lane >> 2) & 3) * 8 + lhalf * 4 + (lane & 3);
     const uint32_t voff_sb = SB1D ? (uint32_t)(min(sb_seg * 64 + lane, b_rows - 1) * p.sfb_sn) * 4u : 0u;
     // Fast-path load of segment seg (8 rows): the segment's first row goes into the
     // wave-uniform SGPR base (clamped to the last valid row), and the lane adds its
@@ -396,7 +420,8 @@ fp8_gemm_1d2d_pipe_kernel(const Fp8GemmArgs p_arg, const int num_m_blocks, const
                 if (part != 2)
                 dma4_saddr(reinterpret_cast<const uint8_t*>(sa_base + (int64_t)kb * p.sfa_sk), voff_sa,
                            stage_lds + SA_OFF + wave * 256);
-            if constexpr (SB1D)
+            if constexpr (SB1D)   // (with the A side: block kb's scales are read after its B side is refilled)
+                if (part != 2)
                 dma4_saddr(reinterpret_cast<const uint8_t*>(sb_base + (int64_t)kb * p.sfb_sk), voff_sb,
                            stage_lds + SB_OFF + sb_seg * 256);
         } else {
@@ -431,7 +456,10 @@ fp8_gemm_1d2d_pipe_kernel(const Fp8GemmArgs p_arg, const int num_m_blocks, const
     i32x8 opB[SN][2], opA[2][2];
     float sa_cur[SM];
     float scl[SPLIT_SB ? SM : 1][SPLIT_SB ? SN : 1];
-    float sbv[SB1D ? SN : 1][SB1D ? 16 : 1];   // SB1D: sb of the lane's 16 columns of each sub-tile
+    // SB1D: sb of the lane's 16 columns of each sub-tile (8q + 4 lhalf + e, the
+    // accumulator layout), column 4q + e of the list in lane 4q + e of each row of
+    // 16 lanes: one register per sub-tile instead of 16.
+    float sbv[SB1D ? SN : 1];
     // sa * sb of the lane's rows for K block kb (read at the top of the block's
     // compute; the stage slot is refilled only after the next barrier).
     auto load_scales = [&](int kb) {
@@ -454,26 +482,31 @@ fp8_gemm_1d2d_pipe_kernel(const Fp8GemmArgs p_arg, const int num_m_blocks, const
             }
         }
         if constexpr (SB1D) {
-            // columns 32j + 8q + 4lhalf + e of the wave's tile (the accumulator layout)
 #pragma unroll
             for (int j = 0; j < SN; ++j)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const f32x4 v = *reinterpret_cast<const f32x4*>(sbase + SB_OFF +
-                                                                    (wn * WN + j * 32 + q * 8 + lhalf * 4) * 4);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) sbv[j][q * 4 + e] = v[e];
-                }
+                sbv[j] = *reinterpret_cast<const float*>(sbase + SB_OFF + (wn * WN + j * 32 + sb_lane) * 4);
         }
     };
     auto scale_of = [&](int i, int j) {
         if constexpr (SPLIT_SB) return scl[i][j];
         else return sa_cur[i];
     };
-    // scale of element e of sub-tile (i, j)
-    auto sc = [&](int i, int j, int e) {
-        if constexpr (SB1D) return sa_cur[i] * sbv[j][e];
-        else return scale_of(i, j);
+    // sub-tile (i, j) of the K block's products into its sums
+    auto promote = [&](int i, int j, const f32x16& acc) {
+        if constexpr (SB1D) {
+            // (an opaque copy: the broadcast lanes are the same for every row
+            // slice, and the compiler would keep all 16 in registers instead of
+            // reading them inside the multiplies)
+            float sb = sbv[j];
+            asm volatile("" : "+v"(sb));
+            promote_bcast4<0>(fin[i][j], acc, sa_cur[i], sb);
+            promote_bcast4<4>(fin[i][j], acc, sa_cur[i], sb);
+            promote_bcast4<8>(fin[i][j], acc, sa_cur[i], sb);
+            promote_bcast4<12>(fin[i][j], acc, sa_cur[i], sb);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 16; ++e) fin[i][j][e] = __builtin_fmaf(scale_of(i, j), acc[e], fin[i][j][e]);
+        }
     };
     auto load_stage_frags = [&](int kb) {
         const uint8_t* sbase = smem + (kb % STAGES) * STAGE_BYTES;
@@ -501,7 +534,7 @@ fp8_gemm_1d2d_pipe_kernel(const Fp8GemmArgs p_arg, const int num_m_blocks, const
     // scale-group load) may stay in flight. Persistent tiles take it too
     // (spill-free with the pinned promotion order below; config-2 shapes as
     // persistent launches 875-880 against 893-899 us).
-    constexpr bool SPLIT = STAGES == 2 && !KT && !SB1D;
+    constexpr bool SPLIT = STAGES == 2 && !KT && (!SB1D || NW == 8);
     // The main loop's MFMA / promotion order: pinned (each sub-tile's MFMA pair,
     // then the previous sub-tile's FMAs) with masks that let LDS, vector-memory
     // and scalar instructions cross, rather than the compiler's interleaving.
@@ -512,7 +545,7 @@ fp8_gemm_1d2d_pipe_kernel(const Fp8GemmArgs p_arg, const int num_m_blocks, const
     // (pinned, the K-grouped launch took 2117-2139 against 2073-2113 us).
     // Persistent tiles take it (config-2 shapes all as persistent launches: 945
     // against 980 us; sparse masked groups 1-2% faster).
-    constexpr bool PIN_PROMO = !SB1D;
+    constexpr bool PIN_PROMO = !SB1D || NW == 4;
     constexpr int kPinMask = 0x7F4;   // SALU, VMEM, DS and transcendental may cross; VALU and MFMA may not
     auto wait_stage = [&](int s) {
         __builtin_amdgcn_sched_barrier(0);
@@ -615,11 +648,7 @@ fp8_gemm_1d2d_pipe_kernel(const Fp8GemmArgs p_arg, const int num_m_blocks, const
                     // promotion FMAs, in that order (the MFMAs and VALU may not cross the
                     // masks; LDS, vector-memory and scalar instructions may).
                     __builtin_amdgcn_sched_barrier(kPinMask);
-                    if (pi >= 0) {
-#pragma unroll
-                        for (int e = 0; e < 16; ++e)
-                            fin[pi][pj][e] = __builtin_fmaf(sc(pi, pj, e), acc[pj][e], fin[pi][pj][e]);
-                    }
+                    if (pi >= 0) promote(pi, pj, acc[pj]);
                     __builtin_amdgcn_sched_barrier(kPinMask);
                 }
                 if (i + 1 == SM) {
@@ -631,11 +660,7 @@ fp8_gemm_1d2d_pipe_kernel(const Fp8GemmArgs p_arg, const int num_m_blocks, const
                 }
                 if constexpr (!PIN_PROMO) {
                     // promote the previous sub-tile
-                    if (pi >= 0) {
-#pragma unroll
-                        for (int e = 0; e < 16; ++e)
-                            fin[pi][pj][e] = __builtin_fmaf(sc(pi, pj, e), acc[pj][e], fin[pi][pj][e]);
-                    }
+                    if (pi >= 0) promote(pi, pj, acc[pj]);
                 }
             }
             if constexpr (PIN_PROMO) {
@@ -651,9 +676,7 @@ fp8_gemm_1d2d_pipe_kernel(const Fp8GemmArgs p_arg, const int num_m_blocks, const
                 }
             }
         }
-#pragma unroll
-        for (int e = 0; e < 16; ++e)
-            fin[SM - 1][SN - 1][e] = __builtin_fmaf(sc(SM - 1, SN - 1, e), acc[SN - 1][e], fin[SM - 1][SN - 1][e]);
+        promote(SM - 1, SN - 1, acc[SN - 1]);
         }
     }
 
@@ -698,17 +721,10 @@ fp8_gemm_1d2d_pipe_kernel(const Fp8GemmArgs p_arg, const int num_m_blocks, const
                                                                                  0, 0, 0, 0);
                         const int pj = j > 0 ? j - 1 : SN - 1;
                         const int pi = j > 0 ? i : i - 1;
-                        if (pi >= 0) {
-#pragma unroll
-                            for (int e = 0; e < 16; ++e)
-                                fin[pi][pj][e] = __builtin_fmaf(sc(pi, pj, e), acc[pj][e], fin[pi][pj][e]);
-                        }
+                        if (pi >= 0) promote(pi, pj, acc[pj]);
                     }
                 }
-#pragma unroll
-                for (int e = 0; e < 16; ++e)
-                    fin[SM - 1][SN - 1][e] =
-                        __builtin_fmaf(sc(SM - 1, SN - 1, e), acc[SN - 1][e], fin[SM - 1][SN - 1][e]);
+                promote(SM - 1, SN - 1, acc[SN - 1]);
             }
         }
     }
@@ -906,16 +922,17 @@ void launch_tile(GemmKind kind, const Fp8GemmArgs& a, hipStream_t stream) {
 
 // 1D1D recipe (SB1D), dense or K-grouped: FP32 D accumulating into C, K (or
 // each group's K) a multiple of 128.
-template <int KIND>
+template <int KIND, int BM, int BN, int WGM, int WGN>
 void launch_1d1d_kind(const Fp8GemmArgs& a, hipStream_t stream) {
-    // 128 x 128 with four waves of 64 x 64 and two stages (217 registers, 68.6 KB
-    // of LDS), so two workgroups share a CU: one's FP32 C/D epilogue, a burst of
-    // HBM traffic with the matrix core idle, runs under the other's K loop
-    // (K-grouped, 8 x 4096 x 7168: 2.02-2.06 ms against 2.17-2.18 ms for 256 x 128
-    // with eight waves and three stages, one workgroup per CU). The per-column
-    // scales (16 more live registers per sub-tile column) do not fit the 256
-    // registers of the eight-wave 256 x 256 tile.
-    constexpr int BM = 128, BN = 128;
+    // 128 x 128: four waves of 64 x 64, two stages (187 registers, 68.6 KB of LDS), so
+    // two workgroups share a CU and one's FP32 C/D epilogue, a burst of HBM traffic
+    // with the matrix core idle, runs under the other's K loop.
+    // 256 x 256: eight waves of 128 x 64, one workgroup per CU, half the L2-to-LDS
+    // bytes per FLOP. The K loop was bound by those bytes: K-grouped, 8 x 4096 x 7168,
+    // K_g ~ 4096, 1582-1596 us with 128 x 128 tiles, 1353-1360 with 256 x 256 (L2-to-LDS
+    // 9.6 and 5.7 TB/s). What is left of it per 256 x 256 tile: about 2.3 us per K
+    // block (the promotion's two VALU operations per element take as long as the
+    // MFMAs) and 21 us of C/D at the HBM rate. The host picks the tile.
     const int num_n_blocks = (a.n + BN - 1) / BN;
     const int num_m_blocks = (a.m + BM - 1) / BM;
     int64_t grid = (int64_t)num_m_blocks * num_n_blocks;
@@ -924,18 +941,22 @@ void launch_1d1d_kind(const Fp8GemmArgs& a, hipStream_t stream) {
     DG_CHECK(grid < (int64_t)1 << 31);
     DG_CHECK(a.out_f32 && a.c != nullptr && a.k % kBK == 0);
     const int raster_gm = choose_raster_gm(BM, BN, num_m_blocks);
-    hipLaunchKernelGGL((fp8_gemm_1d2d_pipe_kernel<BM, BN, 2, 2, 2, KIND, 1, 1, 0, 0, 1>), dim3((unsigned)grid),
-                       dim3(256), 0, stream, a, num_m_blocks, num_n_blocks, raster_gm);
+    hipLaunchKernelGGL((fp8_gemm_1d2d_pipe_kernel<BM, BN, WGM, WGN, 2, KIND, 1, 1, 0, 0, 1>), dim3((unsigned)grid),
+                       dim3(WGM * WGN * 64), 0, stream, a, num_m_blocks, num_n_blocks, raster_gm);
     DG_HIP_CHECK(hipGetLastError());
 }
 
 }  // namespace
 
-void launch_fp8_gemm_1d1d_pipe(bool k_grouped, const Fp8GemmArgs& args, hipStream_t stream) {
-    if (k_grouped)
-        launch_1d1d_kind<kKGrouped>(args, stream);
-    else
-        launch_1d1d_kind<kNormal>(args, stream);
+void launch_fp8_gemm_1d1d_pipe(bool k_grouped, const TileConfig& cfg, const Fp8GemmArgs& args, hipStream_t stream) {
+    const bool big = cfg.block_m == 256;
+    if (k_grouped) {
+        if (big) launch_1d1d_kind<kKGrouped, 256, 256, 2, 4>(args, stream);
+        else launch_1d1d_kind<kKGrouped, 128, 128, 2, 2>(args, stream);
+    } else {
+        if (big) launch_1d1d_kind<kNormal, 256, 256, 2, 4>(args, stream);
+        else launch_1d1d_kind<kNormal, 128, 128, 2, 2>(args, stream);
+    }
 }
 
 bool fp8_1d2d_v2_tile_supported(int bm, int bn) {

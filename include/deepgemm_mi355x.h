@@ -417,7 +417,7 @@ int32_t dg_get_theoretical_mk_alignment_for_contiguous_layout(int32_t expected_m
  * 4 = the pipelined kernel with persistent workgroups (one per CU, striding
  * over the tile sequence like the reference's scheduler; 256 x 256 only),
  * 5 = the weight-streaming kernel (block_m 16 or 160 rows per pass), 6 / 7 =
- * the 1D1D kernels, 8 / 9 = the tiny-M kernel with 8 / 4 waves (block_m = rows
+ * the 1D1D kernels (7: 128 x 128 or 256 x 256), 8 / 9 = the tiny-M kernel with 8 / 4 waves (block_m = rows
  * per workgroup, 16, 32 or 64; block_n = columns per workgroup, 16, 32 or 64),
  * 10 = the split-K kernel of dg_fp8_fp4_gemm_nt_ws (block_m 0; block_n = K
  * chunks, 0 for the heuristic's count);

@@ -228,3 +228,34 @@ def test_k_grouped_chunked_group_order():
         torch.cuda.synchronize()
         assert torch.equal(dd.view(torch.int32), d[g].view(torch.int32)), f'group {g}'
         kb0 += k // 128
+
+
+@pytest.mark.parametrize('ks,m,n', [([128], 256, 256), ([256], 257, 512), ([1152], 511, 264), ([384, 0, 256, 128], 300, 456),
+                                    ([128, 896], 520, 1032)])
+def test_1d1d_256_tile_equals_128(ks, m, n):
+    """The 256 x 256 pipelined 1D1D tile (edges, remainders, one K block, an empty group)
+    computes the bits of the 128 x 128 one, with K- and MN-major scales, and C apart
+    from D or in place."""
+    qa, sfa, qb, sfb, c_np = k_grouped_inputs(ks, m, n, m + n)
+    layout = torch.tensor(ks, dtype=torch.int32, device=DEV)
+    for mn_major in (False, True):
+        sa_t, sb_t = f32(sfa), f32(sfb)
+        if mn_major:
+            sa_t, sb_t = f32(np.ascontiguousarray(sfa.T)).t(), f32(np.ascontiguousarray(sfb.T)).t()
+        outs = []
+        for tile, inplace in ((128, True), (256, True), (256, False)):
+            c = f32(c_np)
+            d = c if inplace else torch.full_like(c, float('nan'))
+            deep_gemm.set_tile_override(tile, tile, variant=7)
+            try:
+                if len(ks) == 1:
+                    a, b = e4m3(qa.reshape(m, -1)), e4m3(qb.reshape(n, -1))
+                    deep_gemm.fp8_gemm_nt((a, sa_t), (b, sb_t), d[0], c=c[0], recipe=(1, 1, 128))
+                else:
+                    deep_gemm.k_grouped_fp8_gemm_nt_contiguous((e4m3(qa), sa_t), (e4m3(qb), sb_t), d, ks, layout, c)
+            finally:
+                deep_gemm.set_tile_override(0, 0)
+            torch.cuda.synchronize()
+            assert f'block_m={tile} ' in deep_gemm.get_last_config()
+            outs.append(d.view(torch.int32))
+        assert torch.equal(outs[1], outs[0]) and torch.equal(outs[2], outs[0])
