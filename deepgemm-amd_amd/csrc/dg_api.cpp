@@ -310,8 +310,9 @@ TileConfig choose_tile_1d2d(GemmKind kind, int64_t m_rows, int64_t n, int64_t k,
     const int tv = g_tile_variant.load(), tm = g_tile_m.load(), tn = g_tile_n.load();
     // The pipelined kernel keeps one SFB value per K block in LDS (up to 1024 blocks).
     const bool pipe_ok = ceil_div(k, 128) <= 1024;
-    // The 256 x 256 pipelined tile is not built for K % 128 != 0 (its K-tail
-    // schedule spills registers); the other tiles give the same bits.
+    // K % 128 != 0: the 256 x 256 pipelined tile is built for dense launches only,
+    // and an override takes it with whole K blocks only (the other tiles give the
+    // same bits).
     const bool tile256_ok = k % 128 == 0;
     if (tv == 4) {   // persistent form of the pipelined kernel
         if (!pipe_ok || tm != 256 || tn != 256) DG_UNSUPPORTED("tile override: the persistent kernel is 256 x 256");
@@ -342,8 +343,7 @@ TileConfig choose_tile_1d2d(GemmKind kind, int64_t m_rows, int64_t n, int64_t k,
     for (const auto& c : cands) {
         if (!grouped_tile_ok(kind, c.variant, c.bm, align_m)) continue;
         if (c.variant == 2 && !pipe_ok) continue;
-        // K % 128 != 0: the 256 x 256 pipelined tile has no K-tail schedule.
-        if (c.variant == 2 && c.bm == 256 && c.bn == 256 && !tile256_ok) continue;
+        if (c.variant == 2 && c.bm == 256 && c.bn == 256 && !tile256_ok && kind != kNormal) continue;
         const int64_t tiles = ceil_div(m_rows, c.bm) * ceil_div(n, c.bn) * groups;
         const int64_t slots = (int64_t)cus * c.per_cu;
         const double rounds = (double)ceil_div(tiles, slots);
@@ -428,7 +428,8 @@ int64_t contiguous_split_rows(int64_t m_rows, int64_t n, int64_t k, int cus, int
 bool is_persistent_route(GemmKind kind, const TileConfig& t, const Fp8GemmArgs& args, int64_t m_rows, int64_t n,
                          int64_t k) {
     if (!(kind == kContiguous || (kind == kNormal && k <= 2048))) return false;
-    if (t.variant != 2 || t.block_m != 256 || t.block_n != 256 || args.out_f32 || args.c != nullptr) return false;
+    if (t.variant != 2 || t.block_m != 256 || t.block_n != 256 || args.out_f32 || args.c != nullptr || k % 128 != 0)
+        return false;
     return ceil_div(m_rows, 256) * ceil_div(n, 256) >= 4 * (int64_t)args.grid_limit;
 }
 

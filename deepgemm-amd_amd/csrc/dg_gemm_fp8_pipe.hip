@@ -26,9 +26,14 @@
 //    g(r) = ((r >> 1) ^ ((r & 1) << 2)) & 7: 16 consecutive rows at one logical
 //    chunk hit distinct banks for 8- and 16-lane LDS phases alike. A lane of the
 //    direct load owns a fixed physical slot and fetches the chunk that belongs there.
-//  * Interior tiles (all rows in range, K a multiple of 128) address every load
-//    as a wave-uniform SGPR base plus one per-lane 32-bit offset; edge tiles
-//    check rows and K chunks and send out-of-range lanes to a zero page.
+//  * Every load is a wave-uniform SGPR base plus one per-lane 32-bit offset, clamped
+//    to the last valid row's last chunk, in interior and edge tiles alike. A partial
+//    last K block (K % 128 != 0) runs after the loop over the whole ones, its
+//    fragments' chunks past K replaced by zeros. (It had a schedule of its own, with
+//    per-lane 64-bit addresses, a zero page and the hand-off at the top of each block:
+//    4096 x 7168 x 2112 101 us on 256 x 192 tiles, 85 with this one, and 71 on the
+//    256 x 256 tile, which has registers for this one only; 3000 x 4400 x 5520 168
+//    and 78.)
 //  * The block's SFB values for all K blocks are loaded into LDS once, so the
 //    main loop issues no vector memory reads besides the stage loads.
 //  * 4 waves in a WGM x WGN grid; wave tile 128 x 64 (or 64 x 64) of 32 x 32
@@ -249,6 +254,7 @@ fp8_gemm_1d2d_pipe_kernel(const Fp8GemmArgs p_arg, const int num_m_blocks, const
     const int a_rows = min(BM, t.row_end - m0);
     const int b_rows = min(BN, p.n - n0);
     const int num_kb = (kdim + kBK - 1) / kBK;
+    const int tail_chunks = (kdim - (num_kb - 1) * kBK) / 16;   // KT: 16-byte chunks of the partial last block
     const int my_group = ((n0 & 127) + wn * WN) >> 7;
 
     // The SFB rows of a tile (at most two 128-row groups of expert `e` from
@@ -329,11 +335,10 @@ fp8_gemm_1d2d_pipe_kernel(const Fp8GemmArgs p_arg, const int num_m_blocks, const
     };
 
     // ---- global -> LDS stage loads
-    // Fast path (K a multiple of 128): one wave-uniform SGPR base per operand and
-    // K block plus a per-lane 32-bit offset. Rows past the tile's valid rows are
-    // clamped to the last valid row: they load a copy of it, and the outputs they
-    // feed (M or N positions past the edge) are never stored.
-    // K-tail path (KT): lanes whose row or K chunk is out of range read a zero page.
+    // One wave-uniform SGPR base per operand and K block plus a per-lane 32-bit
+    // offset. Rows past the tile's valid rows are clamped to the last valid row:
+    // they load a copy of it, and the outputs they feed (M or N positions past the
+    // edge) are never stored.
     // Segment s (8 rows) of a stage is loaded by wave s % NW; since NW is even the
     // swizzle phase of its rows, and so the lane's chunk, is the same for all of a
     // wave's segments. Each load's per-lane offset (row clamped, chunk) is
@@ -347,7 +352,7 @@ fp8_gemm_1d2d_pipe_kernel(const Fp8GemmArgs p_arg, const int num_m_blocks, const
     // SB1D: the column (of 32) whose scale this lane holds
     const int sb_lane = ((lane >> 2) & 3) * 8 + lhalf * 4 + (lane & 3);
     const uint32_t voff_sb = SB1D ? (uint32_t)(min(sb_seg * 64 + lane, b_rows - 1) * p.sfb_sn) * 4u : 0u;
-    // Fast-path load of segment seg (8 rows): the segment's first row goes into the
+    // Load of segment seg (8 rows): the segment's first row goes into the
     // wave-uniform SGPR base (clamped to the last valid row), and the lane adds its
     // own row and chunk, vlane = rs * ld + chunk_off, a loop-invariant register.
     // Lanes past the last valid row are clamped by one v_min_u32 against a uniform
@@ -357,9 +362,14 @@ fp8_gemm_1d2d_pipe_kernel(const Fp8GemmArgs p_arg, const int num_m_blocks, const
     // register across the loop.
     const uint32_t vlane_a = (uint32_t)rs * (uint32_t)lda + chunk_off;
     const uint32_t vlane_b = (uint32_t)rs * (uint32_t)ldb + chunk_off;
-    auto seg_load = [&](const uint8_t* kb_base, int seg, int rows, int64_t ld, uint32_t vlane, uint32_t lds) {
+    // last_chunk: the offset of the K block's last chunk (the partial block of a K
+    // tail: its last one with data, so that no lane reads past the operand's last
+    // row; other rows' lanes past K read the bytes that follow, which the
+    // partial block's fragments replace by zeros).
+    auto seg_load = [&](const uint8_t* kb_base, int seg, int rows, int64_t ld, uint32_t vlane, uint32_t lds,
+                        uint32_t last_chunk = kBK - 16) {
         const int rb = min(seg * 8, rows - 1);
-        uint32_t lim = (uint32_t)(rows - 1 - rb) * (uint32_t)ld + (uint32_t)(kBK - 16);
+        uint32_t lim = (uint32_t)(rows - 1 - rb) * (uint32_t)ld + last_chunk;
         asm volatile("" : "+s"(lim));
         dma16_saddr(kb_base + (int64_t)rb * ld, min(vlane, lim), lds);
     };
@@ -399,55 +409,31 @@ fp8_gemm_1d2d_pipe_kernel(const Fp8GemmArgs p_arg, const int num_m_blocks, const
     // (a literal at every call, folded away once the lambda is inlined)
     auto issue_stage = [&](int kb, int st, int part = 0) {
         const uint32_t stage_lds = smem_lds + st * STAGE_BYTES;
-        if constexpr (!KT) {
-            const uint8_t* a_kb = a_base + (int64_t)kb * kBK;
-            const uint8_t* b_kb = b_base + (int64_t)kb * kBK;
-            if (part != 2) {
+        const uint8_t* a_kb = a_base + (int64_t)kb * kBK;
+        const uint8_t* b_kb = b_base + (int64_t)kb * kBK;
+        const uint32_t last_chunk = KT && kb == num_kb - 1 ? (uint32_t)tail_chunks * 16u - 16u : (uint32_t)(kBK - 16);
+        if (part != 2) {
 #pragma unroll
             for (int i = 0; i < A_INSTR; ++i) {
                 const int seg = i * NW + wave;
-                seg_load(a_kb, seg, a_rows, lda, vlane_a, stage_lds + seg * 1024);
+                seg_load(a_kb, seg, a_rows, lda, vlane_a, stage_lds + seg * 1024, last_chunk);
             }
-            }
-            if (part != 1) {
+        }
+        if (part != 1) {
 #pragma unroll
             for (int i = 0; i < B_INSTR; ++i) {
                 const int seg = i * NW + wave;
-                seg_load(b_kb, seg, b_rows, ldb, vlane_b, stage_lds + BM * kBK + seg * 1024);
+                seg_load(b_kb, seg, b_rows, ldb, vlane_b, stage_lds + BM * kBK + seg * 1024, last_chunk);
             }
-            }
-            if constexpr (!KSA)
-                if (part != 2)
+        }
+        if constexpr (!KSA)
+            if (part != 2)
                 dma4_saddr(reinterpret_cast<const uint8_t*>(sa_base + (int64_t)kb * p.sfa_sk), voff_sa,
                            stage_lds + SA_OFF + wave * 256);
-            if constexpr (SB1D)   // (with the A side: block kb's scales are read after its B side is refilled)
-                if (part != 2)
+        if constexpr (SB1D)   // (with the A side: block kb's scales are read after its B side is refilled)
+            if (part != 2)
                 dma4_saddr(reinterpret_cast<const uint8_t*>(sb_base + (int64_t)kb * p.sfb_sk), voff_sb,
                            stage_lds + SB_OFF + sb_seg * 256);
-        } else {
-#pragma unroll
-            for (int i = 0; i < A_INSTR; ++i) {
-                const int seg = i * NW + wave;
-                const int r = seg * 8 + launder(rs);
-                const int k = kb * kBK + ((pc ^ swz_g(r)) << 4);
-                const void* src = (r < a_rows && k < kdim) ? (const void*)(a_base + (int64_t)r * lda + k)
-                                                          : (const void*)g_zero_page;
-                dma16_vaddr(src, stage_lds + seg * 1024);
-            }
-#pragma unroll
-            for (int i = 0; i < B_INSTR; ++i) {
-                const int seg = i * NW + wave;
-                const int r = seg * 8 + launder(rs);
-                const int k = kb * kBK + ((pc ^ swz_g(r)) << 4);
-                const void* src = (r < b_rows && k < kdim) ? (const void*)(b_base + (int64_t)r * ldb + k)
-                                                          : (const void*)g_zero_page;
-                dma16_vaddr(src, stage_lds + BM * kBK + seg * 1024);
-            }
-            const void* src = (lane < SA_ROWS_PER_WAVE && sa_row < a_rows)
-                                  ? (const void*)(sa_base + (int64_t)sa_row * p.sfa_sm + (int64_t)kb * p.sfa_sk)
-                                  : (const void*)g_zero_page;
-            dma4_vaddr(src, stage_lds + SA_OFF + wave * 256);
-        }
     };
 
     // ---- fragments and scales of a stage
@@ -534,7 +520,7 @@ fp8_gemm_1d2d_pipe_kernel(const Fp8GemmArgs p_arg, const int num_m_blocks, const
     // scale-group load) may stay in flight. Persistent tiles take it too
     // (spill-free with the pinned promotion order below; config-2 shapes as
     // persistent launches 875-880 against 893-899 us).
-    constexpr bool SPLIT = STAGES == 2 && !KT && (!SB1D || NW == 8);
+    constexpr bool SPLIT = STAGES == 2 && (!SB1D || NW == 8);
     // The main loop's MFMA / promotion order: pinned (each sub-tile's MFMA pair,
     // then the previous sub-tile's FMAs) with masks that let LDS, vector-memory
     // and scalar instructions cross, rather than the compiler's interleaving.
@@ -562,7 +548,6 @@ fp8_gemm_1d2d_pipe_kernel(const Fp8GemmArgs p_arg, const int num_m_blocks, const
         __builtin_amdgcn_sched_barrier(0);
     };
 
-    if constexpr (!KT) {
     // Prologue: every slot is free, so the first STAGES stages are issued at once.
     if constexpr (KSA) {
         // group 0 whole (wave w < KSA loads segment w) and segment 0 of group 1
@@ -596,7 +581,8 @@ fp8_gemm_1d2d_pipe_kernel(const Fp8GemmArgs p_arg, const int num_m_blocks, const
     // the registers, so their LDS latency hides under those MFMAs.
     static_assert(SM % 2 == 0, "A fragment double buffer: the next block's first slice goes to buffer 0");
     f32x16 acc[SN];
-    for (int kb = 0; kb < num_kb; ++kb) {
+    const int num_loop = KT ? num_kb - 1 : num_kb;   // the whole blocks
+    for (int kb = 0; kb < num_loop; ++kb) {
         if constexpr (KSA) issue_block_segment(kb);
         if (!wave_computes) {
             if constexpr (SPLIT) {
@@ -680,51 +666,46 @@ fp8_gemm_1d2d_pipe_kernel(const Fp8GemmArgs p_arg, const int num_m_blocks, const
         }
     }
 
-    } else {
-        // K tail: a simpler schedule. The stage loads use per-lane 64-bit
-        // addresses with a zero page for out-of-range chunks, too many live
-        // values to sit inside the MFMA sequence, so the hand-off is at the top of
-        // each block: wait for stage kb (which also certifies that every wave is
-        // done with stage kb - 1), refill that slot, then compute kb.
+    if constexpr (KT) {
+        // The partial last block, after the loop over the whole ones: its stage
+        // landed at the last hand-off, and no stage is issued any more. A
+        // fragment's 16-byte chunks past K become zeros in both operands (what was
+        // loaded there may be anything, NaN codes included).
+        if (wave_computes) {
+            const int kb = num_kb - 1;
+            auto cut = [&](i32x8& f, int ks) {
+                const bool lo = 4 * ks + 2 * lhalf < tail_chunks, hi = 4 * ks + 2 * lhalf + 1 < tail_chunks;
 #pragma unroll
-        for (int s = 0; s < STAGES - 1; ++s)
-            if (s < num_kb) issue_stage(s, s);
-        f32x16 acc[SN];
-        for (int kb = 0; kb < num_kb; ++kb) {
-            __builtin_amdgcn_sched_barrier(0);
-            if constexpr (STAGES == 2) {
-                wait_vmcnt_barrier<0>();
-            } else {
-                if (kb + STAGES - 2 < num_kb)
-                    wait_vmcnt_barrier<(STAGES - 2) * LOADS_PER_STAGE>();
-                else
-                    wait_vmcnt_barrier<0>();
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            if (kb + STAGES - 1 < num_kb) issue_stage(kb + STAGES - 1, (kb + STAGES - 1) % STAGES);
-            if (wave_computes) {
-                load_scales(kb);
-                load_stage_frags(kb);
-                const uint8_t* a_tile = smem + (kb % STAGES) * STAGE_BYTES;
-#pragma unroll
-                for (int i = 0; i < SM; ++i) {
-                    const int cur = i & 1;
-                    if (i + 1 < SM) {
-                        opA[cur ^ 1][0] = frag(a_tile, wm * WM + (i + 1) * 32, 0);
-                        opA[cur ^ 1][1] = frag(a_tile, wm * WM + (i + 1) * 32, 1);
-                    }
-#pragma unroll
-                    for (int j = 0; j < SN; ++j) {
-                        const f32x16 c = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
-                            opB[j][0], opA[cur][0], f32x16{}, 0, 0, 0, 0, 0, 0);
-                        acc[j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(opB[j][1], opA[cur][1], c, 0, 0,
-                                                                                 0, 0, 0, 0);
-                        const int pj = j > 0 ? j - 1 : SN - 1;
-                        const int pi = j > 0 ? i : i - 1;
-                        if (pi >= 0) promote(pi, pj, acc[pj]);
-                    }
+                for (int e = 0; e < 4; ++e) {
+                    f[e] = lo ? f[e] : 0;
+                    f[4 + e] = hi ? f[4 + e] : 0;
                 }
-                promote(SM - 1, SN - 1, acc[SN - 1]);
+            };
+            load_scales(kb);
+            const uint8_t* a_tile = smem + (kb % STAGES) * STAGE_BYTES;
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) {
+#pragma unroll
+                for (int j = 0; j < SN; ++j) cut(opB[j][ks], ks);
+            }
+#pragma unroll
+            for (int i = 0; i < SM; ++i) {
+                const int cur = i & 1;
+                if (i + 1 < SM) {
+                    opA[cur ^ 1][0] = frag(a_tile, wm * WM + (i + 1) * 32, 0);
+                    opA[cur ^ 1][1] = frag(a_tile, wm * WM + (i + 1) * 32, 1);
+                }
+                cut(opA[cur][0], 0);
+                cut(opA[cur][1], 1);
+#pragma unroll
+                for (int j = 0; j < SN; ++j) {
+                    const f32x16 c = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(opB[j][0], opA[cur][0], f32x16{},
+                                                                                     0, 0, 0, 0, 0, 0);
+                    acc[j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(opB[j][1], opA[cur][1], c, 0, 0, 0, 0, 0,
+                                                                             0);
+                    promote(i, j, acc[j]);
+                }
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
     }
@@ -857,12 +838,10 @@ void launch_kind(const Fp8GemmArgs& a, hipStream_t stream) {
     constexpr bool KSA_OK = STAGES == 2 && !PERSIST && (KIND == kNormal || KIND == kContiguous);
     const bool kmajor = KSA_OK && a.sfa_sk == 1 && a.sfa_sm % 4 == 0 && (reinterpret_cast<uintptr_t>(a.sfa) & 15) == 0;
     const int ksa = !kmajor || a.k > kMaxKBlocksKsa * kBK ? 0 : a.k % (4 * kBK) == 0 ? 4 : 0;
-    // The K-tail schedule of the 256 x 256 tile (per-lane 64-bit load addresses next
-    // to 256 registers of accumulators) spills to scratch: it is not built, and
-    // the host never routes a K tail to this tile (K-tail calls take 256 x 192 or
-    // smaller tiles, which compute the same bits).
-    constexpr bool KT_OK = !(BM == 256 && BN == 256);
-    if (k_tail && !KT_OK) DG_UNSUPPORTED("the 256 x 256 pipelined tile needs K % 128 == 0");
+    // K tails: every tile, the 256 x 256 one for dense launches (m-grouped K tails
+    // take 256 x 192 or smaller tiles).
+    constexpr bool KT_OK = !(BM == 256 && BN == 256) || (KIND == kNormal && !PERSIST);
+    if (k_tail && !KT_OK) DG_UNSUPPORTED("this 256 x 256 pipelined tile needs K % 128 == 0");
 #define DG_PIPE_LAUNCH(OF, HC)                                                                                       \
     do {                                                                                                             \
         if (k_tail)                                                                                                  \

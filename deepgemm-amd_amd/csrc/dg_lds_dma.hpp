@@ -10,9 +10,6 @@ namespace dgm {
 namespace dev {
 namespace {
 
-// Source for lanes whose row or K chunk is out of range.
-__device__ __attribute__((aligned(16))) uint8_t g_zero_page[16] = {0};
-
 // Wait until at most N of this wave's vector loads are in flight and its LDS
 // reads have returned, then barrier.
 template <int N>
@@ -53,10 +50,6 @@ __device__ __forceinline__ void dma16_saddr_masked(uint64_t exec_mask, const uin
         : "=&s"(saved)
         : "s"(lds), "v"(voff), "s"(base), "s"(exec_mask)
         : "memory", "m0");
-}
-__device__ __forceinline__ void dma16_vaddr(const void* src, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src)
-                 : "memory", "m0");
 }
 __device__ __forceinline__ void dma4_vaddr(const void* src, uint32_t lds) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(lds), "v"(src)

@@ -107,6 +107,40 @@ def test_all_tiles_bitwise_equal(m, n, k):
         assert torch.equal(o.view(torch.int16), outs[0][1].view(torch.int16))
 
 
+@pytest.mark.parametrize('m,n,k,pad', [(512, 4096, 1040, 112), (300, 520, 144, 0), (257, 264, 16, 16), (200, 320, 2032, 144),
+                                       (2100, 4104, 240, 16), (4000, 7176, 272, 0)])
+def test_k_tail_ignores_what_follows_k(m, n, k, pad):
+    """K % 128 != 0 (one to seven 16-byte chunks in the last block, with and without
+    whole blocks before it): every tile, and the heuristic's own choice (the 256 x 256
+    tile at the larger sizes), gives the bits of the register-staged kernel, whatever
+    follows K in the rows' padding (NaN codes in A and B here)."""
+    x = gen.dense_inputs(m, n, k, seed=m + k)
+    a_buf = torch.full((m, k + pad), 0x7F, dtype=torch.uint8, device=DEV)
+    b_buf = torch.full((n, k + pad), 0xFF, dtype=torch.uint8, device=DEV)
+    a_buf[:, :k] = gen.to_dev(x['qa'])
+    b_buf[:, :k] = gen.to_dev(x['qb'])
+    a = (a_buf[:, :k].view(torch.float8_e4m3fn), f32(x['sfa']))
+    b = (b_buf[:, :k].view(torch.float8_e4m3fn), f32(x['sfb']))
+    outs, cfgs = [], []
+    for v, bm, bn in ((1, 64, 64), (0, 0, 0), (2, 128, 128), (2, 128, 256), (2, 256, 128), (2, 256, 192)):
+        deep_gemm.set_tile_override(bm, bn, variant=v)
+        try:
+            d = sentinel_bf16((m, n))
+            deep_gemm.fp8_gemm_nt(a, b, d)
+            cfgs.append(deep_gemm.get_last_config())
+        finally:
+            deep_gemm.set_tile_override(0, 0)
+        outs.append(d.view(torch.int16))
+    torch.cuda.synchronize()
+    print(f'k-tail m={m} n={n} k={k}: {cfgs[1]}', flush=True)
+    if m == 4000:
+        assert 'block_m=256 block_n=256' in cfgs[1], cfgs[1]
+    for o, c in zip(outs[1:], cfgs[1:]):
+        assert torch.equal(o, outs[0]), c
+    ref = ogemm.gemm_nt(oquant.dequant_per_token(x['qa'], x['sfa'])[:64], oquant.dequant_per_block(x['qb'], x['sfb']))
+    assert ogemm.calc_diff(outs[1].view(torch.bfloat16)[:64].float().cpu().numpy(), ref) < 1e-3
+
+
 @pytest.mark.parametrize('m,n,k,acc', [(4096, 7168, 4096, False), (4096, 7168, 4096, True), (8192, 7168, 4096, False),
                                         (4096, 7040, 4096, False)])   # the 256 x 192 launch ends in a 64-column tile
 def test_dense_column_split_equals_one_launch(m, n, k, acc):
