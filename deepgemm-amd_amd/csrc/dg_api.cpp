@@ -338,9 +338,12 @@ TileConfig choose_tile_1d2d(GemmKind kind, int64_t m_rows, int64_t n, int64_t k,
         {1, 128, 128, 2, 0.80}, {1, 128, 64, 3, 0.55}, {1, 64, 128, 3, 0.55}, {1, 64, 64, 4, 0.45}};
     int cus = 256;
     try { cus = num_sms_now(); } catch (const Error&) {}
+    const bool whole_k_contiguous = kind == kContiguous && k % 128 == 0 && align_m % 128 == 0 && groups <= kMaxTabGroups;
     double best = 1e300;
     TileConfig out{64, 64, 1};
     for (const auto& c : cands) {
+        // (256-row tiles of these calls: the block table's, is_table_route)
+        if (whole_k_contiguous && c.bm == 256) continue;
         if (!grouped_tile_ok(kind, c.variant, c.bm, align_m)) continue;
         if (c.variant == 2 && !pipe_ok) continue;
         if (c.variant == 2 && c.bm == 256 && c.bn == 256 && !tile256_ok && kind != kNormal) continue;
@@ -384,23 +387,23 @@ int64_t dense_split_columns(int64_t m_rows, int64_t n, int64_t k, int cus) {
     return best < 0.95 * whole ? best_n1 : 0;
 }
 
-// Row split of an m-grouped contiguous call (m_indices layout) whose 256 x 256
-// tiles leave the last round mostly empty (8 experts, 32768 tokens, N = 4096:
-// 131 M blocks x 16 = 2096 tiles, 8 full rounds and 48 tiles): rows [0, r1) run
-// as 256 x 256 tiles and rows [r1, M) as smaller tiles (there 192 tiles of
-// 128 x 128, each a quarter of the work). r1 is a multiple of 256 and segments
-// start on the M alignment, so each part is itself an m_indices layout; every
-// tile shape computes its outputs with the same arithmetic, so the result is
-// bitwise that of one launch. Returns r1 and the second launch's tile, or 0 when
-// the per-round cost model gains less than 5% or K is under 4096 (as for the
-// column split). With 256-column tiles only (the fused SwiGLU epilogue) the bar
-// is 3%: config 3's gate/up launch, 2096 tiles, split into 2048 tiles of
-// 256 x 256 and 80 of 128 x 256 for a modelled 3.5% (measured 1097 -> 1083 us).
-// In launches of four rounds or more the first part takes the persistent walk
-// (is_persistent_route) when it still makes four rounds.
-int64_t contiguous_split_rows(int64_t m_rows, int64_t n, int64_t k, int cus, int align_m, TileConfig& hi_tile,
-                              bool bn256_only = false) {
+// Row split of an m-grouped contiguous call (m_indices layout) whose 256 x 256 tiles
+// leave the last round nearly empty (35 M blocks x 16: 2 rounds and 48 tiles): rows
+// [0, r1) run as 256 x 256 tiles and rows [r1, M) as smaller ones. r1 is a multiple of
+// 256 and segments start on the M alignment, so each part is itself an m_indices
+// layout; every tile shape computes its outputs with the same arithmetic, so the
+// result is bitwise that of one launch. Returns r1 and the second launch's tile, or
+// 0 when the last round is more than 3/16 full, the per-round cost model gains less
+// than 11% or K is under 4096. Since the persistent walk cuts tiles from the segments'
+// own starts and leaves padding blocks out (its rounds no longer follow from M), one
+// launch is the faster one wherever the split was measured against it (8 experts, us,
+// split / one launch: 9216 x 4096 x 4096 205 / 183, 16768 x 4096 x 4096 321 / 308,
+// 33792 x 4096 x 7168 1013 / 982), so the split is bounded to the launches that it was
+// built for.
+int64_t contiguous_split_rows(int64_t m_rows, int64_t n, int64_t k, int cus, int align_m, TileConfig& hi_tile) {
     if (k < 4096) return 0;
+    const int64_t left = ceil_div(m_rows, 256) * ceil_div(n, 256) % cus;
+    if (left == 0 || 16 * left > 3 * (int64_t)cus) return 0;
     struct Part { int bm, bn; double eff; };
     static const Part parts[] = {{256, 128, 1.00}, {128, 256, 0.97}, {128, 128, 0.80}};   // as in choose_tile_1d2d
     constexpr double t256 = 256.0 * 256 / 1.32;
@@ -413,24 +416,38 @@ int64_t contiguous_split_rows(int64_t m_rows, int64_t n, int64_t k, int cus, int
     for (int64_t mb1 = mb - 1; mb1 >= 1; --mb1)
         for (const auto& p : parts) {
             if (!grouped_tile_ok(kContiguous, 2, p.bm, align_m)) continue;
-            if (bn256_only && p.bn != 256) continue;
             const int64_t rows2 = m_rows - mb1 * 256;
             const double cost = rounds(mb1 * ceil_div(n, 256)) * t256 +
                                 rounds(ceil_div(rows2, p.bm) * ceil_div(n, p.bn)) * (p.bm * p.bn / p.eff);
             if (cost < best - 1e-9) best = cost, best_r1 = mb1 * 256, hi_tile = TileConfig{p.bm, p.bn, 2};
         }
-    return best < (bn256_only ? 0.97 : 0.95) * whole ? best_r1 : 0;
+    return best < 0.89 * whole ? best_r1 : 0;
 }
 
-// Whether a dense or contiguous call on 256 x 256 tiles runs as persistent
-// workgroups (variant 4): BF16 D without C, at least four rounds of tiles on
-// the CUs, and for dense calls K <= 2048 (measurements in run_gemm).
+// Whether a dense call on 256 x 256 tiles runs as persistent workgroups (variant 4):
+// BF16 D without C, at least four rounds of tiles on the CUs and K <= 2048
+// (measurements in run_gemm).
 bool is_persistent_route(GemmKind kind, const TileConfig& t, const Fp8GemmArgs& args, int64_t m_rows, int64_t n,
                          int64_t k) {
-    if (!(kind == kContiguous || (kind == kNormal && k <= 2048))) return false;
+    if (kind != kNormal || k > 2048) return false;
     if (t.variant != 2 || t.block_m != 256 || t.block_n != 256 || args.out_f32 || args.c != nullptr || k % 128 != 0)
         return false;
     return ceil_div(m_rows, 256) * ceil_div(n, 256) >= 4 * (int64_t)args.grid_limit;
+}
+
+// Whether an m-grouped contiguous call (m_indices layout) runs the persistent
+// 256 x 256 walk over its block table: whole K blocks, and more 128 x 256 tiles than
+// CUs (up to one round of those is faster as such). Measured against the fastest
+// other tile (us, 128 x 256 -> persistent): 4 experts 1536 x 4096 x 7168 (192 tiles)
+// 81 -> 110; 2560 x 4096 x 4096 (320) 76 -> 63, 2048 x 7168 x 2048 (448) 49 -> 45,
+// 5120 x 4096 x 4096 136 -> 120, 32 experts 12288 x 4096 x 7168 502 -> 380, 36864 x
+// 7168 x 2048 766 -> 589; slower only where every segment is one block (16 experts
+// 4096 x 4096 x 2048 53 -> 63, but 32 experts 5120 x 4096 x 2048 80 -> 66). One
+// workgroup per 256-row tile at multiples of 256 rows took 515 and 606 us on the two
+// 32-expert calls.
+bool is_table_route(int64_t m_rows, int64_t n, int64_t k, int64_t groups, int cus, int align_m) {
+    return k % 128 == 0 && ceil_div(k, 128) <= 1024 && align_m % 128 == 0 && groups <= kMaxTabGroups &&
+           ceil_div(m_rows, 128) * ceil_div(n, 256) > cus;
 }
 
 void record_config(const char* kernel, GemmKind kind, const TileConfig& t, int64_t m, int64_t n, int64_t k,
@@ -665,12 +682,12 @@ void run_gemm(GemmKind kind, const Operands& o, const Recipe& r, int64_t m, int6
             // workgroup's start and first-stage wait once per tile, the persistent
             // walk once per CU. Measured per launch (µs, per tile -> persistent):
             // 4096 x 24576 x 1536 (6 rounds) 170-173 -> 168-172 (K-major SFA 195 ->
-            // 189); contiguous 33408 x 7168 x 2048 (14 rounds) 522-524 -> 509-510,
-            // 33408 x 4096 x 7168 (8 rounds, per tile with the row split) 958-961 ->
-            // 942-943. Dense calls with longer K are even (within 1-2% at 4-8
+            // 189). Dense calls with longer K are even (within 1-2% at 4-8
             // rounds) and keep the per-tile launch and its column split; at 1-3.5
             // rounds it loses (4096 x 7168 x 2048 +5%), and with FP32 C it is even.
             if (tv == 0 && is_persistent_route(kind, t, args, m_rows, n, k)) t.variant = 4;
+            if (tv == 0 && kind == kContiguous && is_table_route(m_rows, n, k, groups, args.grid_limit, align_m))
+                t = {256, 256, 4};
         }
         if (!grouped_tile_ok(kind, t.variant, t.block_m, align_m))
             DG_UNSUPPORTED("M alignment for contiguous layout must be a multiple of 64");
@@ -694,12 +711,7 @@ void run_gemm(GemmKind kind, const Operands& o, const Recipe& r, int64_t m, int6
                 return;
             }
         }
-        // (persistent launches too: their last round is as uneven; the first rows
-        // stay persistent when they still make four rounds. Measured, interleaved
-        // bench runs: 33408 x 4096 x 7168 970-981 -> 954-958 us, the first 32768
-        // rows 880-890 us and the 640-row tail on 128 x 128 tiles 43 us.)
-        if (kind == kContiguous && tv == 0 && (t.variant == 2 || t.variant == 4) && t.block_m == 256 &&
-            t.block_n == 256) {
+        if (kind == kContiguous && tv == 0 && t.variant == 4) {
             TileConfig ht{};
             const int64_t r1 = contiguous_split_rows(m_rows, n, k, args.grid_limit, align_m, ht);
             if (r1 > 0) {
@@ -707,10 +719,7 @@ void run_gemm(GemmKind kind, const Operands& o, const Recipe& r, int64_t m, int6
                                  std::to_string(ht.block_n);
                 Fp8GemmArgs lo = args;
                 lo.m = (int32_t)r1;
-                TileConfig lt = t;
-                if (lt.variant == 4 && !is_persistent_route(kind, TileConfig{256, 256, 2}, args, r1, n, k))
-                    lt.variant = 2;
-                launch_fp8_gemm_1d2d_v2(kind, lt, lo, stream);
+                launch_fp8_gemm_1d2d_v2(kind, t, lo, stream);
                 // rows [r1, m): A rows, SFA rows (K- or MN-major: sfa_sm is the row
                 // stride), m_indices entries and D rows
                 Fp8GemmArgs hi = args;
@@ -1032,9 +1041,9 @@ void swiglu_l1_impl(GemmKind kind, const dg_tensor* a_, const dg_tensor* sfa_, c
     args.sw_clamp = clamp > 0.f ? clamp : 0.f;
 
     // Tile: the 256-column tiles of the pipelined kernel (256 rows when K % 128 == 0
-    // and the layout allows, else 128; for masked groups far below max_m the
-    // persistent 256 x 256 walk), or for masked decode groups the weight-streaming
-    // kernel with 8 waves (256 columns).
+    // and the layout allows, else 128; the persistent 256 x 256 walk for masked groups
+    // far below max_m, and for contiguous calls of more than a round of 128-row tiles),
+    // or for masked decode groups the weight-streaming kernel with 8 waves (256 columns).
     const int tv = g_tile_variant.load(), tm = g_tile_m.load(), tn = g_tile_n.load();
     const bool ktail = k % 128 != 0;
     if (ceil_div(k, 128) > 1024) DG_UNSUPPORTED("fused SwiGLU: K up to 131072");
@@ -1058,8 +1067,10 @@ void swiglu_l1_impl(GemmKind kind, const dg_tensor* a_, const dg_tensor* sfa_, c
         t = {kMaskedStreamRows, 256, 5};
     } else if (masked && t.block_m == 256 && ceil_div(m, 256) >= 2 * ceil_div(std::max(expected_m, 1), 256)) {
         t.variant = 4;   // the persistent group walk, as for the plain masked launch (run_gemm)
-    } else if (kind == kContiguous && is_persistent_route(kind, t, args, m, n, k)) {
-        t.variant = 4;   // many rounds of tiles: persistent, as the plain contiguous launch (run_gemm)
+    } else if (kind == kContiguous && is_table_route(m, n, k, g, args.grid_limit, align_m)) {
+        t.variant = 4;   // the persistent walk over the block table, as the plain contiguous launch (run_gemm)
+    } else if (kind == kContiguous) {
+        t.block_m = 128;   // (at most one round of 128 x 256 tiles, or a K tail)
     }
     if (t.variant == 2 && !grouped_tile_ok(kind, 2, t.block_m, align_m))
         DG_UNSUPPORTED("M alignment for contiguous layout must be a multiple of 128 for the fused SwiGLU epilogue");
@@ -1067,31 +1078,6 @@ void swiglu_l1_impl(GemmKind kind, const dg_tensor* a_, const dg_tensor* sfa_, c
     if (t.variant == 5) {
         launch_fp8_gemm_masked_stream(args, 8, false, stream);
         return;
-    }
-    if (kind == kContiguous && tv == 0 && (t.variant == 2 || t.variant == 4) && t.block_m == 256) {
-        // the row split of the plain contiguous launch, with a 256-column second tile
-        TileConfig ht{};
-        const int64_t r1 = contiguous_split_rows(m, n, k, args.grid_limit, align_m, ht, true);
-        if (r1 > 0) {
-            t_last_config += " split_m=" + std::to_string(r1) + ":" + std::to_string(ht.block_m) + "x" +
-                             std::to_string(ht.block_n);
-            Fp8GemmArgs lo = args;
-            lo.m = (int32_t)r1;
-            TileConfig lt = t;
-            if (lt.variant == 4 && !is_persistent_route(kind, TileConfig{256, 256, 2}, args, r1, n, k))
-                lt.variant = 2;
-            launch_fp8_gemm_1d2d_v2(kind, lt, lo, stream);
-            Fp8GemmArgs hi = args;
-            hi.m = (int32_t)(m - r1);
-            hi.a = args.a + r1 * args.lda;
-            hi.sfa = args.sfa + r1 * args.sfa_sm;
-            hi.layout = args.layout + r1;
-            hi.sw_q = args.sw_q + r1 * args.sw_ldq;
-            hi.sw_sf = args.sw_sf + r1 * args.sw_sf_sm;
-            if (args.sw_w) hi.sw_w = args.sw_w + r1;
-            launch_fp8_gemm_1d2d_v2(kind, ht, hi, stream);
-            return;
-        }
     }
     launch_fp8_gemm_1d2d_v2(kind, t, args, stream);
 }

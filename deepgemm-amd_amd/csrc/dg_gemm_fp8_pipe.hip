@@ -149,6 +149,20 @@ fp8_gemm_1d2d_pipe_kernel(const Fp8GemmArgs p_arg, const int num_m_blocks, const
     __shared__ __attribute__((aligned(16))) float s_sag[KSA ? 3 : 1][KSA ? BM : 1][KSA ? KSA : 1];   // [slot][row][kb % KSA]
     __shared__ int s_flag;
     __shared__ int s_half_valid[2];
+    // persistent contiguous launches: the block table and its counts
+    constexpr bool TAB = PERSIST && KIND == kContiguous;
+    static_assert(!TAB || BM == 256, "block table of 256- and 128-row tiles");
+    __shared__ uint32_t s_tab[TAB ? (EPI ? kMaxTabBlocksEpi : kMaxTabBlocks) : 1];
+    __shared__ int s_tab_n[2];
+    // the SwiGLU epilogue's table: 256-row tiles keep it beside the ring (filled once
+    // per workgroup), 128-row ones fill it behind their staged rows
+    __shared__ float s_silu[EPI && BM == 256 ? SiluTable::kEntries : 1];
+    if constexpr (EPI && BM == 256) SiluTable::fill<NT>(s_silu, threadIdx.x);   // (read after the K loop's barriers)
+    if constexpr (TAB) {
+        static_assert(STAGES * STAGE_BYTES >= 4 * kMaxTabBlocks, "the table's scratch fits the stage ring");
+        build_block_table<NT>(p_arg.layout, p_arg.m, p_arg.num_groups, reinterpret_cast<uint32_t*>(smem), s_tab, s_tab_n);
+        __syncthreads();
+    }
 
     // PF: persistent two-stage launches issue the next tile's SFB and first stage
     // into stage slot 0 during this tile's epilogue, which then stages its outputs
@@ -175,9 +189,13 @@ fp8_gemm_1d2d_pipe_kernel(const Fp8GemmArgs p_arg, const int num_m_blocks, const
     PTile t{};
     if constexpr (PERSIST) {
         if (lt != slot) __syncthreads();   // every wave is done with the previous tile's LDS
-        t = decode_tile_persistent<BM, BN, KIND, NT>(lt, p.m, p.n, p.num_groups, p.layout, p.align_m, p.zero_padding,
-                                                     num_m_blocks, num_n_blocks, static_cast<uint16_t*>(p.d), p.ldd,
-                                                     &s_flag, raster_gm);
+        if constexpr (TAB)
+            t = table_tile_coords<BN>(lt, p.m, s_tab, __builtin_amdgcn_readfirstlane(s_tab_n[0]),
+                                      __builtin_amdgcn_readfirstlane(s_tab_n[1]), num_n_blocks, raster_gm);
+        else
+            t = decode_tile_persistent<BM, BN, KIND, NT>(lt, p.m, p.n, p.num_groups, p.layout, p.align_m, p.zero_padding,
+                                                         num_m_blocks, num_n_blocks, static_cast<uint16_t*>(p.d), p.ldd,
+                                                         raster_gm);
         if constexpr (PF) {
             // (a tile is only prefetched when it exists and has rows; were that
             // ever wrong, its loads are drained here rather than left writing LDS)
@@ -215,7 +233,7 @@ fp8_gemm_1d2d_pipe_kernel(const Fp8GemmArgs p_arg, const int num_m_blocks, const
     // those rows are stored.
     int npass = 1;
     int pass_expert[2] = {t.expert, t.expert};
-    if constexpr (KIND == kContiguous && BM > 128) {
+    if constexpr (KIND == kContiguous && BM > 128 && !TAB) {
         static_assert(BM == 256 && 128 % WM == 0, "two 128-row blocks, each a whole number of wave rows");
         if (tid < 2) s_half_valid[tid] = 0;
         __syncthreads();
@@ -287,7 +305,7 @@ fp8_gemm_1d2d_pipe_kernel(const Fp8GemmArgs p_arg, const int num_m_blocks, const
     // waves per SIMD. readfirstlane: the value is wave-uniform and the compiler
     // must see it so, or code merged below the branch gets per-lane LDS addresses.)
     bool wave_computes;
-    if constexpr (KIND == kMasked)
+    if constexpr (KIND == kMasked || TAB)
         wave_computes = __builtin_amdgcn_readfirstlane((int)(wm * WM < a_rows && p.m >= 0)) != 0;
     else
         wave_computes = (npass == 1 || (wm * WM) >> 7 == pass) && p.m >= 0;
@@ -739,14 +757,22 @@ fp8_gemm_1d2d_pipe_kernel(const Fp8GemmArgs p_arg, const int num_m_blocks, const
                 for (int q = 0; q < 4; ++q)
                     Buf::put4(smem, wm * WM + i * 32 + lrow, wn * WN + j * 32 + q * 8 + lhalf * 4, fin[i][j][q * 4],
                               fin[i][j][q * 4 + 1], fin[i][j][q * 4 + 2], fin[i][j][q * 4 + 3]);
+        float* silu = s_silu;
+        if constexpr (BM != 256) {
+            static_assert(STAGES * STAGE_BYTES >= Buf::kBytes + SiluTable::kBytes, "table behind the staged rows");
+            silu = reinterpret_cast<float*>(smem + Buf::kBytes);
+            SiluTable::fill<NT>(silu, wave * 64 + lane);
+        }
         __syncthreads();
         const int m_lo = npass == 2 ? m0 + pass * 128 : m0;
-        const int m_hi = npass == 2 ? m_lo + 128 : m0 + BM;
+        const int m_hi = TAB ? t.row_end : npass == 2 ? m_lo + 128 : m0 + BM;
         const SwigluOut o{p.sw_q, p.sw_ldq, p.sw_q_gs, p.sw_sf, p.sw_sf_sm, p.sw_sf_sk,
                           p.sw_sf_gs, p.sw_w, p.sw_w_gs, p.sw_clamp};
-        Buf::template run<NW>(smem, wave, lane, m0, KIND == kMasked ? t.g : 0, n0 >> 8, o,
-                              [&](int m, bool& st, bool& z) {
-                                  row_predicate<KIND>(t, p.m, p.layout, m, st, z);
+        Buf::template run<NW>(smem, silu, wave, lane, m0, KIND == kMasked ? t.g : 0, n0 >> 8, o, p.m - 1,
+                              [&](int m) { return KIND == kContiguous ? p.layout[min(m, p.m - 1)] : 0; },
+                              [&](int m, int id, bool& st, bool& z) {
+                                  if constexpr (KIND == kContiguous) st = m < p.m && id >= 0, z = false;
+                                  else row_predicate<KIND>(t, p.m, p.layout, m, st, z);
                                   if (m < m_lo || m >= m_hi) st = z = false;
                               });
     } else {
@@ -758,7 +784,7 @@ fp8_gemm_1d2d_pipe_kernel(const Fp8GemmArgs p_arg, const int num_m_blocks, const
         const void* c_g = (KIND == kKGrouped && HAS_C) ? (const void*)(static_cast<const float*>(p.c) + (int64_t)t.g * p.c_gs)
                                                        : p.c;
         const int m_lo = npass == 2 ? m0 + pass * 128 : m0;
-        const int m_hi = npass == 2 ? m_lo + 128 : m0 + BM;
+        const int m_hi = TAB ? t.row_end : npass == 2 ? m_lo + 128 : m0 + BM;
         if constexpr (PF) {
             // The next tile's SFB and stage 0 (into slot 0, as its prologue would
             // issue them), issued once the first rows are staged: they arrive while
@@ -797,7 +823,7 @@ fp8_gemm_1d2d_pipe_kernel(const Fp8GemmArgs p_arg, const int num_m_blocks, const
     };   // run_pass
 
     run_pass(0);
-    if constexpr (KIND == kContiguous && BM > 128) {
+    if constexpr (KIND == kContiguous && BM > 128 && !TAB) {
         if (npass == 2) run_pass(1);
     }
     if constexpr (!PERSIST) break;
@@ -827,6 +853,8 @@ void launch_kind(const Fp8GemmArgs& a, hipStream_t stream) {
     if (grid == 0) return;
     DG_CHECK(grid < (int64_t)1 << 31);
     DG_CHECK((a.k + kBK - 1) / kBK <= kMaxKBlocks);
+    if (PERSIST && KIND == kContiguous)   // (the block table holds up to one tile per 128 rows)
+        grid = (int64_t)((a.m + 127) / 128) * num_n_blocks;
     if (PERSIST) grid = std::min<int64_t>(grid, std::max(1, a.grid_limit));
     const int raster_gm = choose_raster_gm(BM, BN, num_m_blocks);
     const dim3 gdim(static_cast<unsigned>(grid)), bdim(WGM * WGN * 64);
@@ -866,11 +894,7 @@ void launch_kind(const Fp8GemmArgs& a, hipStream_t stream) {
                 hipLaunchKernelGGL((fp8_gemm_1d2d_pipe_kernel<BM, BN, WGM, WGN, STAGES, KIND, 0, 0, KT_OK ? 1 : 0, 0, 0,
                                                               0, 1>),
                                    gdim, bdim, 0, stream, a, num_m_blocks, num_n_blocks, raster_gm);
-            else if (ksa == 4)
-                hipLaunchKernelGGL((fp8_gemm_1d2d_pipe_kernel<BM, BN, WGM, WGN, STAGES, KIND, 0, 0, 0, 0, 0,
-                                                              KSA_OK ? 4 : 0, 1>),
-                                   gdim, bdim, 0, stream, a, num_m_blocks, num_n_blocks, raster_gm);
-            else
+            else   // (no scale groups: their ring would take the SiLU table's LDS)
                 hipLaunchKernelGGL((fp8_gemm_1d2d_pipe_kernel<BM, BN, WGM, WGN, STAGES, KIND, 0, 0, 0, 0, 0, 0, 1>),
                                    gdim, bdim, 0, stream, a, num_m_blocks, num_n_blocks, raster_gm);
         } else {
@@ -947,6 +971,30 @@ void launch_fp8_gemm_1d2d_v2(GemmKind kind, const TileConfig& cfg, const Fp8Gemm
     const int key = cfg.block_m * 1000 + cfg.block_n;
     if (cfg.variant == 4) {   // persistent workgroups
         if (key != 256256) DG_UNSUPPORTED("the persistent pipelined kernel is compiled for 256 x 256 tiles only");
+        if (kind == kContiguous && args.num_groups > kMaxTabGroups) {   // (the same bits, one workgroup per tile)
+            launch_tile<256, 256, 2, 4, 2>(kind, args, stream);
+            return;
+        }
+        const int64_t max_rows = (args.sw_q ? kMaxTabBlocksEpi : kMaxTabBlocks) * (int64_t)128;
+        if (kind == kContiguous && args.m > max_rows) {
+            // rows in launches of as many 128-row blocks as the block table holds: each
+            // range is an m_indices layout of its own
+            for (int64_t r0 = 0; r0 < args.m; r0 += max_rows) {
+                Fp8GemmArgs part = args;
+                part.m = (int32_t)std::min<int64_t>(args.m - r0, max_rows);
+                part.a = args.a + r0 * args.lda;
+                part.sfa = args.sfa + r0 * args.sfa_sm;
+                part.layout = args.layout + r0;
+                if (args.d) part.d = static_cast<uint8_t*>(args.d) + r0 * args.ldd * 2;   // BF16 (checked at the launch)
+                if (args.sw_q) {
+                    part.sw_q = args.sw_q + r0 * args.sw_ldq;
+                    part.sw_sf = args.sw_sf + r0 * args.sw_sf_sm;
+                    if (args.sw_w) part.sw_w = args.sw_w + r0;
+                }
+                launch_tile<256, 256, 2, 4, 2, 1>(kind, part, stream);
+            }
+            return;
+        }
         launch_tile<256, 256, 2, 4, 2, 1>(kind, args, stream);
         return;
     }

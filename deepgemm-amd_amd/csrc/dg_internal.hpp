@@ -124,6 +124,12 @@ bool fp8_splitk_supported(const Fp8GemmArgs& a);
 SplitKPlan plan_fp8_splitk(int64_t m, int64_t n, int64_t k, int cus, int splits);
 void launch_fp8_gemm_splitk(const Fp8GemmArgs& a, const SplitKPlan& plan, float* ws, hipStream_t stream);
 
+// Persistent contiguous launches: 128-row blocks of one launch (longer calls run as
+// several), and groups, that fit the block table's entries and LDS.
+constexpr int kMaxTabBlocks = 4096;
+constexpr int kMaxTabBlocksEpi = 504;   // with the SwiGLU epilogue's table in LDS
+constexpr int kMaxTabGroups = 65535;
+
 // Launch the FP32-scale FP8 GEMM for `kind` with tile `cfg` on `stream`.
 // Throws dgm::Error on unsupported configurations or launch failures.
 void launch_fp8_gemm_1d2d(GemmKind kind, const TileConfig& cfg, const Fp8GemmArgs& args,

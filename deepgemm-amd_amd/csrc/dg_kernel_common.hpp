@@ -236,22 +236,113 @@ __device__ __forceinline__ PTile persistent_tile_coords(int lt, int m, int num_g
     return t;
 }
 
+// ---- the contiguous layout's block table (persistent launches)
+//
+// 256-row tiles at multiples of 256 rows straddle two experts wherever a segment
+// has an odd number of 128-row blocks, and such a tile runs twice, each time
+// with half of its waves idle. The persistent kernel cuts the segments themselves
+// instead: a run of consecutive blocks of one expert becomes 256-row tiles from
+// the run's start and at most one 128-row tile. Every workgroup builds the table of
+// its launch once (blocks without a row to store are left out), and no tile reads
+// m_indices to find its expert.
+// Entry: 128-row block index, expert << 16. Entries [0, nf) are the 256-row tiles,
+// [nf, nf + nh) the 128-row ones: the tile sequence holds all columns of the former
+// first, so that the short ones fill the last round.
+// NT threads, at least one wave; tmp: ceil(m / 128) words of scratch LDS. The caller
+// syncs before reading. The expert of a block is max(0, m_indices[its first row]),
+// clamped to the last group; a block with no row to store is left out.
+template <int NT>
+__device__ __forceinline__ void build_block_table(const int32_t* __restrict__ layout, int m, int num_groups,
+                                                  uint32_t* tmp, uint32_t* tab, int* counts) {
+    constexpr uint32_t kNone = 0xFFFFFFFFu;
+    constexpr int UN = 8;   // wave loads of 256 rows in flight
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int nblk = (m + 127) >> 7;
+    const int npair = (nblk + 1) >> 1;
+    const bool aligned = (reinterpret_cast<uintptr_t>(layout) & 15) == 0;
+    for (int p0 = wave; p0 < npair; p0 += UN * (NT / 64)) {
+        i32x4 v[UN];
+#pragma unroll
+        for (int q = 0; q < UN; ++q) {
+            // (rows past m repeat the last ones; their blocks' entries are cut below)
+            const int row = (p0 + q * (NT / 64)) * 256 + lane * 4;
+            if (aligned && row + 4 <= m) {
+                v[q] = *reinterpret_cast<const i32x4*>(layout + row);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[q][e] = row + e < m ? layout[row + e] : -1;
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < UN; ++q) {
+            const uint64_t any = __ballot((v[q][0] & v[q][1] & v[q][2] & v[q][3]) >= 0);   // any id >= 0
+            const int blk = (p0 + q * (NT / 64)) * 2 + (lane >> 5);
+            const bool valid = (lane >> 5 ? any >> 32 : any & 0xFFFFFFFFu) != 0;
+            if ((lane & 31) == 0 && blk < nblk)
+                tmp[blk] = valid ? (uint32_t)min(max(0, v[q][0]), num_groups - 1) : kNone;
+        }
+    }
+    __syncthreads();
+    if (wave != 0) return;
+    // Fulls to tab from the front, halves behind all of them: counted first.
+    int nf = 0, nh = 0, n_full = 0;
+    for (int pass = 0; pass < 2; ++pass) {
+        int run = 0;   // first block of the run that reaches into this chunk
+        nf = 0, nh = 0;
+        for (int base = 0; base < nblk; base += 64) {
+            const int i = base + lane;
+            const uint32_t e = i < nblk ? tmp[i] : kNone;
+            const uint32_t before = i > 0 && i < nblk ? tmp[i - 1] : kNone;
+            const uint32_t after = i + 1 < nblk ? tmp[i + 1] : kNone;
+            const uint64_t starts = __ballot(e != before);
+            const uint64_t below = starts & (~0ull >> (63 - lane));   // starts at lanes <= this one
+            const int first = below ? base + 63 - __builtin_clzll(below) : run;
+            const bool emit = e != kNone && ((i - first) & 1) == 0;
+            const uint64_t fm = __ballot(emit && after == e), hm = __ballot(emit && after != e);
+            const uint64_t lt = (1ull << lane) - 1;
+            if (pass == 1 && emit) {
+                const int pos = after == e ? nf + __popcll(fm & lt) : n_full + nh + __popcll(hm & lt);
+                tab[pos] = (uint32_t)i | e << 16;
+            }
+            nf += __popcll(fm), nh += __popcll(hm);
+            if (starts) run = base + 63 - __builtin_clzll(starts);
+        }
+        n_full = nf;
+    }
+    if (lane == 0) counts[0] = nf, counts[1] = nh;
+}
+
+// Tile lt of the launch's sequence from the block table; done past its end.
+template <int BN>
+__device__ __forceinline__ PTile table_tile_coords(int lt, int m, const uint32_t* tab, int nf, int nh, int num_n_blocks,
+                                                   int raster_gm) {
+    PTile t{};
+    const int fulls = nf * num_n_blocks;
+    const bool full = lt < fulls;
+    if (lt >= fulls + nh * num_n_blocks) {
+        t.done = 1;
+        return t;
+    }
+    int mb, nb;
+    raster_tile(full ? lt : lt - fulls, full ? nf : nh, num_n_blocks, raster_gm, mb, nb);
+    const uint32_t entry = __builtin_amdgcn_readfirstlane(tab[full ? mb : nf + mb]);
+    t.m0 = (int)(entry & 0xFFFFu) * 128;
+    t.n0 = nb * BN;
+    t.expert = (int)(entry >> 16);
+    t.row_end = min(m, t.m0 + (full ? 256 : 128));
+    t.active = 1;
+    return t;
+}
+
 template <int BM, int BN, int KIND, int NT>
 __device__ __forceinline__ PTile decode_tile_persistent(int lt, int m, int n, int num_groups,
                                                         const int32_t* __restrict__ layout, int align_m,
                                                         int zero_padding, int num_m_blocks, int num_n_blocks,
-                                                        uint16_t* zero_d, int64_t ldd, int* s_flag, int raster_gm) {
+                                                        uint16_t* zero_d, int64_t ldd, int raster_gm) {
+    static_assert(KIND != kContiguous, "contiguous launches walk a block table");
     PTile t = persistent_tile_coords<BM, BN, KIND>(lt, m, num_groups, layout, num_m_blocks, num_n_blocks, raster_gm);
     if (t.done) return t;
-    if constexpr (KIND == kContiguous) {
-        t.expert = min(max(0, layout[t.m0]), num_groups - 1);
-        if (threadIdx.x == 0) *s_flag = 0;
-        __syncthreads();
-        for (int r = threadIdx.x; r < BM; r += NT)
-            if (t.m0 + r < m && layout[t.m0 + r] >= 0) *s_flag = 1;
-        __syncthreads();
-        t.active = *s_flag;
-    } else if constexpr (KIND == kPsum) {
+    if constexpr (KIND == kPsum) {
         int gi = 0, end = 0, aend = 0;
         for (; gi < num_groups; ++gi) {
             end = layout[gi];

@@ -90,6 +90,66 @@ __device__ __forceinline__ float swiglu_weighted(float g, float u, float w, floa
     return f32_mul(f32_mul(silu_f32(g), u), w);
 }
 
+// silu_f32 of every BF16 value with 2^-10 <= |g| < 2^8, for an LDS table: the exact
+// steps of silu_f32 cost about 45 operations a value, and the tile's phase 2 was
+// bound by them (18 us of a 256 x 256 tile, 12 of them here), while a gate is one of
+// these 4608 values almost always. Entry 2 (magnitude bits - kLo) + sign; kThreads
+// threads fill it once per workgroup (9 values each of 512).
+struct SiluTable {
+    static constexpr uint32_t kLo = 0x3A80, kHi = 0x4380;   // BF16 bits of 2^-10, 2^8
+    static constexpr uint32_t kEntries = 2 * (kHi - kLo);
+    static constexpr int kBytes = kEntries * 4;
+    template <int NT>
+    __device__ static void fill(float* table, int tid) {
+        for (uint32_t i = tid; i < kEntries; i += NT)
+            table[i] = silu_f32(__uint_as_float((kLo + (i >> 1)) << 16 | i << 31));
+    }
+};
+
+// y = silu(gate) * up * w of one lane's eight packed BF16 gates and ups (the bits of
+// swiglu_weighted), silu from the table, the values outside it computed.
+__device__ __forceinline__ void swiglu8(const uint32_t (&gw)[4], const uint32_t (&uw)[4], float w, float clamp,
+                                        const float* table, float (&y)[8]) {
+    typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+    constexpr unsigned short kBase = 2 * SiluTable::kLo, kLast = SiluTable::kEntries - 1;
+    u16x2 idx[4], top{0, 0};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const u16x2 b = __builtin_bit_cast(u16x2, gw[i]);
+        idx[i] = (b << 1 | b >> 15) - kBase;   // outside the table: past its end
+        top = __builtin_elementwise_max(top, idx[i]);
+    }
+    float s[8];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t off = __builtin_bit_cast(uint32_t, __builtin_elementwise_min(idx[i], u16x2{kLast, kLast}) << 2);
+        const char* t = reinterpret_cast<const char*>(table);
+        s[2 * i] = *reinterpret_cast<const float*>(t + (off & 0xFFFFu));
+        s[2 * i + 1] = *reinterpret_cast<const float*>(t + (off >> 16));
+    }
+    static_assert(SiluTable::kBytes <= 65536, "16-bit byte offsets");
+    if (__builtin_expect(__ballot(top.x > kLast || top.y > kLast) != 0, 0)) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            if ((e & 1 ? idx[e >> 1].y : idx[e >> 1].x) > kLast)
+                s[e] = silu_f32(__uint_as_float(e & 1 ? gw[e >> 1] & 0xFFFF0000u : gw[e >> 1] << 16));
+    }
+    if (clamp > 0.f) {   // a gate above it (or NaN) counts as the clamp
+        const float sc = silu_f32(clamp);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const float g = __uint_as_float(e & 1 ? gw[e >> 1] & 0xFFFF0000u : gw[e >> 1] << 16);
+            s[e] = g <= clamp ? s[e] : sc;
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        float u = __uint_as_float(e & 1 ? uw[e >> 1] & 0xFFFF0000u : uw[e >> 1] << 16);
+        if (clamp > 0.f) u = fminf(clamp, fmaxf(-clamp, u));
+        y[e] = f32_mul(f32_mul(s[e], u), w);
+    }
+}
+
 // OCP e4m3 code of v by explicit rounding (saturating to 0x7F | sign past 464,
 // NaN -> 0x7F | sign): the path for groups whose amax is not finite.
 __device__ __forceinline__ uint32_t e4m3_code_slow(float v) {
@@ -106,6 +166,11 @@ __device__ __forceinline__ uint32_t e4m3_code_slow(float v) {
     return sign | (uint32_t)rintf(r * 512.0f);
 }
 
+template <int CTRL>
+__device__ __forceinline__ float dpp_f32(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+
 // The per-token quantizer over one lane's 8 consecutive values, the group being
 // TPG adjacent lanes (TPG = GRAN / 8). Every lane of the wave must call it (the
 // amax exchange and the finiteness vote are wave-wide). Returns the 8 codes
@@ -115,8 +180,15 @@ __device__ __forceinline__ uint2 quantize_group8(const float (&y)[8], float& sf_
     float amax = 0.f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(y[e]));
-#pragma unroll
-    for (int o = TPG / 2; o > 0; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o));
+    // over the group's TPG lanes, by DPP within each row of 16 lanes (a maximum does
+    // not depend on the order): lanes ^ 1, ^ 2, mirrored in 8, mirrored in 16
+    static_assert(TPG == 4 || TPG == 16, "quads or whole rows of lanes");
+    amax = fmaxf(amax, dpp_f32<0xB1>(amax));
+    amax = fmaxf(amax, dpp_f32<0x4E>(amax));
+    if constexpr (TPG == 16) {
+        amax = fmaxf(amax, dpp_f32<0x141>(amax));
+        amax = fmaxf(amax, dpp_f32<0x140>(amax));
+    }
     amax = fmaxf(amax, 1e-4f);
     const float sf = f32_mul(amax, 1.0f / 448.0f);
     const float inv = __fdiv_rn(1.0f, sf);
@@ -174,30 +246,46 @@ struct SwigluTile {
     // columns [8 (lane & 15), +8) of the tile. Row r is output row row0 + r of
     // group g; it is quantized and stored when `store` holds, and written as
     // a zero row (zero codes, the scale of an all-zero group) when `zero`
-    // holds (pred(row, store, zero) sets both; zero is ignored when store holds).
+    // holds (pred(row, fetched, store, zero) sets both; zero is ignored when store holds).
     // ib: the tile's intermediate column block (q columns [128 ib, +128)).
-    template <int NW, typename Pred>
-    __device__ static void run(const uint8_t* buf, int wave, int lane, int row0, int g, int ib, const SwigluOut& o,
-                               Pred pred) {
+    // fetch(row) loads what pred needs of a row (clamped to the rows that exist) and
+    // is called, with the row's weight, one step ahead of its use: each was a
+    // global round trip on every step's path. last_row: the last row of w. table: a
+    // filled SiluTable, or null.
+    template <int NW, typename Fetch, typename Pred>
+    __device__ static void run(const uint8_t* buf, const float* table, int wave, int lane, int row0, int g, int ib,
+                               const SwigluOut& o, int last_row, Fetch fetch, Pred pred) {
         static_assert(ROWS % (4 * NW) == 0, "whole row groups per wave");
         const int c16 = lane & 15;
+        const int r_first = wave * 4 + (lane >> 4);
+        auto weight = [&](int m) { return o.w ? o.w[(int64_t)g * o.w_gs + min(m, last_row)] : 1.f; };
+        int raw_next = fetch(row0 + r_first);
+        float w_next = weight(row0 + r_first);
 #pragma unroll 1
-        for (int r = wave * 4 + (lane >> 4); r < ROWS; r += 4 * NW) {
+        for (int r = r_first; r < ROWS; r += 4 * NW) {
             const int m = row0 + r;
-            bool st, z;
-            pred(m, st, z);
             const uint4 gv = *reinterpret_cast<const uint4*>(buf + offset(r, 8 * c16));
             const uint4 uv = *reinterpret_cast<const uint4*>(buf + offset(r, 128 + 8 * c16));
-            const uint32_t gw[4] = {gv.x, gv.y, gv.z, gv.w}, uw[4] = {uv.x, uv.y, uv.z, uv.w};
+            const int raw = raw_next;
+            const float w = w_next;
+            raw_next = fetch(m + 4 * NW);
+            w_next = weight(m + 4 * NW);
+            bool st, z;
+            pred(m, raw, st, z);
             z = z && !st;
-            const float w = (st && o.w) ? o.w[(int64_t)g * o.w_gs + m] : 1.f;
+            const uint32_t gw[4] = {gv.x, gv.y, gv.z, gv.w}, uw[4] = {uv.x, uv.y, uv.z, uv.w};
             float y[8];
+            if (table) {
+                swiglu8(gw, uw, w, o.clamp, table, y);
+            } else {
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float gf = bf16_to_f32(static_cast<uint16_t>(e & 1 ? gw[e >> 1] >> 16 : gw[e >> 1] & 0xFFFFu));
-                const float uf = bf16_to_f32(static_cast<uint16_t>(e & 1 ? uw[e >> 1] >> 16 : uw[e >> 1] & 0xFFFFu));
-                y[e] = st ? swiglu_weighted(gf, uf, w, o.clamp) : 0.f;
+                for (int e = 0; e < 8; ++e)
+                    y[e] = swiglu_weighted(__uint_as_float(e & 1 ? gw[e >> 1] & 0xFFFF0000u : gw[e >> 1] << 16),
+                                           __uint_as_float(e & 1 ? uw[e >> 1] & 0xFFFF0000u : uw[e >> 1] << 16), w,
+                                           o.clamp);
             }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) y[e] = st ? y[e] : 0.f;
             float sf;
             const uint2 codes = quantize_group8<16>(y, sf);
             if (st || z) {

@@ -1454,3 +1454,71 @@ def test_fp4_equals_converted_fp8():
     assert diff < 1e-9
     assert neq.mean() < 0.01
     assert worst <= 2 ** -9 * scale
+
+
+def _table_layout(case):
+    """(m_indices, groups) of a contiguous layout that exercises the block table."""
+    def seg(*parts):   # (expert, rows, blocks)
+        out = []
+        for e, r, b in parts:
+            out += [e] * r + [-1] * (b * 128 - r)
+        return np.array(out, np.int32)
+    if case == 'odd_even_runs':   # runs of 1, 2, 3, 4 and 5 blocks, an expert without rows, one in two runs
+        return seg((0, 100, 1), (2, 256, 2), (3, 300, 3), (0, 512, 4), (4, 600, 5), (5, 1, 1)), 6
+    if case == 'padding_blocks':   # blocks without a row inside and after the segments
+        return seg((0, 130, 2), (1, 0, 1), (1, 128, 1), (1, 0, 3), (2, 200, 4)), 3
+    if case == 'first_row_padding':   # a block's expert is max(0, its first row's id)
+        x = seg((0, 128, 1), (1, 256, 2), (2, 128, 1))
+        x[128:140] = -1
+        return x, 3
+    if case == 'ids_past_last':
+        return seg((0, 128, 1), (7, 256, 2), (1, 90, 1)), 2
+    if case == 'all_padding':
+        return seg((0, 0, 5)), 2
+    if case == 'ragged_end':   # the last block is cut
+        return seg((0, 256, 2), (1, 256, 2), (1, 128, 1))[:-55], 2
+    assert case == 'two_launches'   # more 128-row blocks than one table holds
+    return np.concatenate([np.full(128 * 4095, 0, np.int32), np.full(128 * 3, 1, np.int32)]), 2
+
+
+@pytest.mark.parametrize('case', ['odd_even_runs', 'padding_blocks', 'first_row_padding', 'ids_past_last', 'all_padding',
+                                  'ragged_end', 'two_launches'])
+@pytest.mark.parametrize('shift', [0, 1])
+def test_contiguous_block_table(case, shift):
+    """The persistent contiguous walk over its block table (variant 4) equals one
+    workgroup per 128-row tile bit for bit and leaves the same rows alone, also with
+    m_indices 4 bytes off a 16-byte boundary, and with fewer CUs than tiles."""
+    idx, g = _table_layout(case)
+    m, n, k = len(idx), 256 if case == 'two_launches' else 520, 128 if case == 'two_launches' else 256
+    print(f'block table {case} shift={shift} m={m}', flush=True)
+    dg = torch.Generator(device=DEV).manual_seed(5)
+    a = deep_gemm.per_token_cast_to_fp8(torch.randn((m, k), generator=dg, device=DEV).bfloat16(), use_ue8m0=False)
+    w = [deep_gemm.per_block_cast_to_fp8(torch.randn((n, k), generator=dg, device=DEV).bfloat16(), use_ue8m0=False)
+         for _ in range(g)]
+    b = (torch.stack([q.view(torch.uint8) for q, _ in w]).view(torch.float8_e4m3fn), torch.stack([s for _, s in w]))
+    gl = torch.zeros(m + shift, dtype=torch.int32, device=DEV)[shift:]
+    gl.copy_(torch.from_numpy(idx))
+    outs = []
+    for v, bm, bn, cus in ((2, 128, 128, 0), (4, 256, 256, 0), (4, 256, 256, 3)):
+        before = deep_gemm.get_num_sms()
+        deep_gemm.set_tile_override(bm, bn, variant=v)
+        if cus:
+            deep_gemm.set_num_sms(cus)
+        try:
+            d = sentinel_bf16((m, n))
+            deep_gemm.m_grouped_fp8_gemm_nt_contiguous(a, b, d, gl)
+        finally:
+            deep_gemm.set_tile_override(0, 0)
+            deep_gemm.set_num_sms(before)
+        outs.append(d.view(torch.int16))
+    torch.cuda.synchronize()
+    assert torch.equal(outs[1], outs[0]) and torch.equal(outs[2], outs[0])
+    assert bool((outs[1][gl < 0] == SENTINEL).all())
+    if case != 'all_padding':
+        rows = np.nonzero(idx >= 0)[0][[0, -1]]
+        e = np.minimum(np.maximum(idx[rows // 128 * 128], 0), g - 1)
+        for r, ei in zip(rows, e):
+            ref = ogemm.gemm_nt(oquant.dequant_per_token(a[0][r:r + 1].view(torch.uint8).cpu().numpy(),
+                                                         a[1][r:r + 1].cpu().numpy()),
+                                oquant.dequant_per_block(b[0][ei].view(torch.uint8).cpu().numpy(), b[1][ei].cpu().numpy()))
+            assert ogemm.calc_diff(outs[1][r:r + 1].view(torch.bfloat16).float().cpu().numpy(), ref) < 1e-3

@@ -355,3 +355,45 @@ def test_moe_layer_fused_end_to_end():
     assert diff < 1e-3
     for key, val in outs.items():
         assert torch.equal(val.view(torch.int16), outs[('contiguous', False)].view(torch.int16)), key
+
+
+@pytest.mark.parametrize('rows_per_expert,experts', [(700, 3), (16500, 4), (90, 5)])
+@pytest.mark.parametrize('clamp', [None, 7.0])
+def test_fused_gate_range(rows_per_expert, experts, clamp):
+    """Gates of every magnitude (rows scaled by 2^-40 .. 2^60, zero rows, rows that
+    overflow to Inf and NaN) through the epilogue's table and past both of its ends:
+    fused == unfused bit for bit, on 128- and 256-row tiles, and over more blocks
+    than one launch's table holds (4 x 16500 rows)."""
+    inter, k = 256, 128
+    aligned = (rows_per_expert + 127) // 128 * 128
+    rows = aligned * experts
+    print(f'gate range rows={rows} clamp={clamp}', flush=True)
+    dg = torch.Generator(device=DEV).manual_seed(11)
+    x = torch.randn((rows, k), generator=dg, device=DEV).bfloat16()
+    qa, sfa = deep_gemm.per_token_cast_to_fp8(x, use_ue8m0=False)
+    r = torch.arange(rows, device=DEV)
+    sfa = sfa * torch.exp2((r % 51 * 2 - 40).float())[:, None]
+    sfa[r % 53 == 7] = 0.0
+    sfa[r % 59 == 9] = 3e38
+    m_idx = (r // aligned).int()
+    m_idx[r % aligned >= rows_per_expert] = -1
+    w = _weights(experts, 2 * inter, k, 70)
+    wf = deep_gemm.transform_l1_weights_for_swiglu(w)
+    rw = torch.rand((rows,), generator=dg, device=DEV)
+    h = torch.empty((rows, 2 * inter), dtype=torch.bfloat16, device=DEV)
+    deep_gemm.m_grouped_fp8_gemm_nt_contiguous((qa, sfa), w, h, m_idx)
+    rq, rsf = deep_gemm.moe_swiglu_apply_weight_to_fp8(h, rw, m_idx, clamp_value=clamp)
+    stored = (m_idx >= 0).cpu().numpy()
+    for tile in (None, (256, 256), (128, 256)):
+        q, sf = _alloc_out((rows,), inter)
+        if tile:
+            deep_gemm.set_tile_override(*tile, variant=2)
+        try:
+            deep_gemm.m_grouped_fp8_gemm_nt_contiguous_swiglu((qa, sfa), wf, (q, sf), m_idx, rw, activation_clamp=clamp)
+            cfg = deep_gemm.get_last_config()
+        finally:
+            deep_gemm.set_tile_override(0, 0)
+        torch.cuda.synchronize()
+        if tile is None and rows > 65536:
+            assert ' v4 ' in cfg, cfg
+        _check_rows(q, sf, rq, rsf, stored)
