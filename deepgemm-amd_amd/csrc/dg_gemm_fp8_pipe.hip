@@ -128,7 +128,7 @@ fp8_gemm_1d2d_pipe_kernel(const Fp8GemmArgs p_arg, const int num_m_blocks, const
     constexpr int KSA_LPR = KSA ? KSA / 4 : 1;         // lanes per row (16 bytes each)
     constexpr int KSA_RPS = 64 / KSA_LPR;              // rows per 1 KB segment of a group
     // one segment per K block of the group, a 64-lane segment split over the waves
-    static_assert(!KSA || (STAGES == 2 && !KT && !SB1D && !PERSIST && BM / KSA_RPS == KSA && NW == 8),
+    static_assert(!KSA || (STAGES == 2 && !KT && !SB1D && (!PERSIST || KIND == kContiguous) && BM / KSA_RPS == KSA && NW == 8),
                   "K-major SFA groups");
     // When every wave's N range sits in one 128-row SFB block, sa and sb fold into
     // one factor per row; otherwise (e.g. 192-wide tiles) each 32-column sub-tile
@@ -860,10 +860,12 @@ void launch_kind(const Fp8GemmArgs& a, hipStream_t stream) {
     const dim3 gdim(static_cast<unsigned>(grid)), bdim(WGM * WGN * 64);
     const bool k_tail = (a.k % kBK) != 0;
     // K-major SFA scale groups (one 16-byte load of a row's scales per 4 K blocks).
+    // Persistent contiguous launches too (K-major, 8 experts 33792 x 4096 x 7168 998 ->
+    // 920 us, 32 experts 12288 x 4096 x 7168 376 -> 341, K = 2048 within 2%).
     // The kernel also takes groups of 8 (32 bytes); with the split hand-off the
     // groups of 4 measured faster (dense 929 against 952 us over the config-2
     // shapes, and the contiguous kernel spills with 8).
-    constexpr bool KSA_OK = STAGES == 2 && !PERSIST && (KIND == kNormal || KIND == kContiguous);
+    constexpr bool KSA_OK = STAGES == 2 && (PERSIST ? KIND == kContiguous : KIND == kNormal || KIND == kContiguous);
     const bool kmajor = KSA_OK && a.sfa_sk == 1 && a.sfa_sm % 4 == 0 && (reinterpret_cast<uintptr_t>(a.sfa) & 15) == 0;
     const int ksa = !kmajor || a.k > kMaxKBlocksKsa * kBK ? 0 : a.k % (4 * kBK) == 0 ? 4 : 0;
     // K tails: every tile, the 256 x 256 one for dense launches (m-grouped K tails

@@ -126,7 +126,7 @@ void launch_fp8_gemm_splitk(const Fp8GemmArgs& a, const SplitKPlan& plan, float*
 
 // Persistent contiguous launches: 128-row blocks of one launch (longer calls run as
 // several), and groups, that fit the block table's entries and LDS.
-constexpr int kMaxTabBlocks = 4096;
+constexpr int kMaxTabBlocks = 3072;
 constexpr int kMaxTabBlocksEpi = 504;   // with the SwiGLU epilogue's table in LDS
 constexpr int kMaxTabGroups = 65535;
 
