@@ -5,6 +5,9 @@ host API (*.cpp) is plain C++ compiled by g++ against the HIP runtime headers.
 All objects are linked by hipcc into deep_gemm/libdeepgemm_mi355x.so next to the
 Python package, so the library travels with the source tree.
 
+The native half of the Python binding (bind/dg_bind.cpp) is compiled by g++ against
+torch's headers into deep_gemm/_dgbind.so, a CPython module.
+
 Usage: python deepgemm-amd_amd/csrc/build.py [--jobs N] [--verbose]
 """
 import argparse
@@ -19,6 +22,8 @@ PKG = os.path.dirname(HERE)
 ROOT = os.path.dirname(PKG)
 INCLUDE = os.path.join(ROOT, 'include')
 OBJ_DIR = os.path.join(PKG, '_build')
+BIND_SRC = os.path.join(HERE, 'bind', 'dg_bind.cpp')
+BIND_PATH = os.path.join(PKG, 'deep_gemm', '_dgbind.so')
 LIB_PATH = os.path.join(PKG, 'deep_gemm', 'libdeepgemm_mi355x.so')
 ROCM = os.environ.get('ROCM_PATH', '/opt/rocm')
 HIPCC = os.path.join(ROCM, 'bin', 'hipcc')
@@ -61,14 +66,35 @@ def _compile(src, verbose):
     return obj
 
 
+def build_bind(verbose=False):
+    import sysconfig
+    import torch
+    root = os.path.dirname(torch.__file__)
+    inc = os.path.join(root, 'include')
+    tmp = BIND_PATH + '.tmp'
+    cmd = ['g++', '-O2', '-std=c++17', '-fPIC', '-shared', '-Wall', '-D_GLIBCXX_USE_CXX11_ABI=' +
+           str(int(torch._C._GLIBCXX_USE_CXX11_ABI)), '-I', INCLUDE, '-isystem', inc, '-isystem',
+           os.path.join(inc, 'torch', 'csrc', 'api', 'include'), '-isystem', sysconfig.get_paths()['include'], BIND_SRC,
+           '-o', tmp, '-L', os.path.join(root, 'lib'), '-ltorch_python', '-ltorch_cpu', '-lc10']
+    if verbose:
+        print(' '.join(cmd), flush=True)
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f'compile failed: {BIND_SRC}\n{res.stderr}')
+    os.replace(tmp, BIND_PATH)
+    return BIND_PATH
+
+
 def build(jobs=None, verbose=False):
     if not os.path.exists(HIPCC):
         raise RuntimeError(f'hipcc not found at {HIPCC}')
     os.makedirs(OBJ_DIR, exist_ok=True)
     srcs = sources()
     jobs = jobs or min(len(srcs), max(1, (os.cpu_count() or 4)))
-    with cf.ThreadPoolExecutor(max_workers=jobs) as ex:
+    with cf.ThreadPoolExecutor(max_workers=jobs + 1) as ex:
+        bind = ex.submit(build_bind, verbose)
         objs = list(ex.map(lambda s: _compile(s, verbose), srcs))
+        bind.result()
     tmp = LIB_PATH + '.tmp'
     cmd = [HIPCC, '--offload-arch=' + ARCH, '-shared', '-fPIC', '-o', tmp] + objs
     if verbose:
@@ -82,8 +108,9 @@ def build(jobs=None, verbose=False):
 
 def clean():
     shutil.rmtree(OBJ_DIR, ignore_errors=True)
-    if os.path.exists(LIB_PATH):
-        os.remove(LIB_PATH)
+    for path in (LIB_PATH, BIND_PATH):
+        if os.path.exists(path):
+            os.remove(path)
 
 
 if __name__ == '__main__':

@@ -19,7 +19,8 @@ import ctypes
 import torch
 
 from . import _ffi
-from ._ffi import check as _check, describe as _desc, ref as _ref
+from ._ffi import address as _address, bind as _bind, check as _check, describe as _desc
+from ._ffi import raw_stream_of as _raw_stream_of, ref as _ref
 
 __version__ = '2.8.1+mi355x'
 
@@ -209,25 +210,12 @@ def fp8_fp4_gemm_nt(a: Tuple[torch.Tensor, torch.Tensor], b: Tuple[torch.Tensor,
     ep, fp8q = _resolve_epilogue(epilogue, alpha)
     a_t, sfa = _pair(a, 'a')
     b_t, sfb = _pair(b, 'b')
-    da, dsa, db, dsb = _desc(a_t), _desc(sfa), _desc(b_t), _desc(sfb)
-    dc = _desc(c) if c is not None else None
     r = _ffi.recipe_struct(recipe, recipe_a, recipe_b)
 
     def run(out):
-        dd = _desc(out)
-        # Decode-sized calls (at most 64 rows) split K over workgroups when given a
-        # workspace: it comes from torch's caching allocator on the output's stream.
-        ws_bytes = 0
-        if c is None and a_t.dim() == 2 and a_t.shape[0] <= 64 and out.dtype == torch.bfloat16:
-            ws_bytes = int(_lib.dg_fp8_gemm_nt_workspace_size(a_t.shape[0], b_t.shape[0], a_t.shape[1]))
-        if ws_bytes > 0:
-            ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=out.device)
-            _check(_lib.dg_fp8_fp4_gemm_nt_ws(_ref(da), _ref(dsa), _ref(db), _ref(dsb), _ref(dd), _ref(dc), _ref(r),
-                                              int(bool(disable_ue8m0_cast)), _ref(ep), _ref(_desc(ws)),
-                                              _ffi.stream_of(out)))
-        else:
-            _check(_lib.dg_fp8_fp4_gemm_nt(_ref(da), _ref(dsa), _ref(db), _ref(dsb), _ref(dd), _ref(dc), _ref(r),
-                                           int(bool(disable_ue8m0_cast)), _ref(ep), _ffi.stream_of(out)))
+        # (calls of at most 64 rows get their split-K workspace there)
+        _check(_bind.gemm_nt(a_t, sfa, b_t, sfb, out, c, _address(r), int(bool(disable_ue8m0_cast)), _address(ep),
+                             _raw_stream_of(out)))
     if fp8q is not None:
         _fp8_quantized_output(d, c, a_t.shape[-1], fp8q, run)
     else:
@@ -268,13 +256,11 @@ def m_grouped_fp8_fp4_gemm_nt_contiguous(a, b, d: torch.Tensor, grouped_layout: 
         raise RuntimeError('Unsupported error: the FP8Quantization epilogue takes the dense GEMM here')
     a_t, sfa = _pair(a, 'a')
     b_t, sfb = _pair(b, 'b')
-    da, dsa, db, dsb, dd, dl = _desc(a_t), _desc(sfa), _desc(b_t), _desc(sfb), _desc(d), _desc(grouped_layout)
     r = _ffi.recipe_struct(recipe, recipe_a, recipe_b)
-    _check(_lib.dg_m_grouped_fp8_fp4_gemm_nt_contiguous(
-        _ref(da), _ref(dsa), _ref(db), _ref(dsb), _ref(dd), _ref(dl), _ref(r), int(bool(disable_ue8m0_cast)),
-        int(bool(use_psum_layout)), int(bool(ensure_zero_padding)),
-        -1 if expected_m_for_psum_layout is None else int(expected_m_for_psum_layout), _ref(ep),
-        _ffi.stream_of(d)))
+    _check(_bind.contiguous(a_t, sfa, b_t, sfb, d, grouped_layout, _address(r), int(bool(disable_ue8m0_cast)),
+                            int(bool(use_psum_layout)), int(bool(ensure_zero_padding)),
+                            -1 if expected_m_for_psum_layout is None else int(expected_m_for_psum_layout),
+                            _address(ep), _raw_stream_of(d)))
 
 
 def m_grouped_fp8_fp4_gemm_nn_contiguous(a, b, d, grouped_layout, recipe=None, recipe_a=None, recipe_b=None,
@@ -297,11 +283,9 @@ def m_grouped_fp8_fp4_gemm_nt_masked(a, b, d: torch.Tensor, masked_m: torch.Tens
         raise RuntimeError('Unsupported error: the FP8Quantization epilogue takes the dense GEMM here')
     a_t, sfa = _pair(a, 'a')
     b_t, sfb = _pair(b, 'b')
-    da, dsa, db, dsb, dd, dm = _desc(a_t), _desc(sfa), _desc(b_t), _desc(sfb), _desc(d), _desc(masked_m)
     r = _ffi.recipe_struct(recipe, recipe_a, recipe_b)
-    _check(_lib.dg_m_grouped_fp8_fp4_gemm_nt_masked(
-        _ref(da), _ref(dsa), _ref(db), _ref(dsb), _ref(dd), _ref(dm), int(expected_m), _ref(r),
-        int(bool(disable_ue8m0_cast)), _ref(ep), _ffi.stream_of(d)))
+    _check(_bind.masked(a_t, sfa, b_t, sfb, d, masked_m, int(expected_m), _address(r), int(bool(disable_ue8m0_cast)),
+                        _address(ep), _raw_stream_of(d)))
 
 
 def _k_grouped(entry, a, b, d, ks_cpu, grouped_layout, c, recipe, use_psum_layout, epilogue):
@@ -459,18 +443,13 @@ def per_token_cast_to_fp8(x: torch.Tensor, use_ue8m0: bool, gran_k: int = 128,
         sf = torch.empty((m, (groups + 3) // 4), dtype=torch.int32, device=x.device)
     else:
         sf = torch.empty((m, groups), dtype=torch.float32, device=x.device)
-    _check(_lib.dg_per_token_cast_to_fp8(_ref(_desc(x)), _ref(_desc(q)), _ref(_desc(sf)), int(gran_k),
-                                         int(bool(use_ue8m0)), _ffi.stream_of(x)))
+    _check(_bind.cast(x, q, sf, int(gran_k), int(bool(use_ue8m0)), _raw_stream_of(x)))
     return q, sf
 
 
 # ------------------------------------------------------------------ MoE plumbing
 
 _MOE_LAYOUTS = {'contiguous': 0, 'psum': 1, 'masked': 2}
-
-
-def _opt(t):
-    return _ref(_desc(t)) if t is not None else None
 
 
 def moe_dispatch(x: Tuple[torch.Tensor, torch.Tensor], topk_idx: torch.Tensor, num_experts: int,
@@ -513,9 +492,8 @@ def moe_dispatch(x: Tuple[torch.Tensor, torch.Tensor], topk_idx: torch.Tensor, n
     w = torch.empty((rows,), dtype=torch.float32, device=dev) if topk_weights is not None else None
     ws_bytes = int(_lib.dg_moe_dispatch_workspace_size(int(t), int(num_experts)))
     ws = torch.empty((max(ws_bytes, 4) // 4,), dtype=torch.int32, device=dev)
-    _check(_lib.dg_moe_dispatch(_ref(_desc(xq)), _ref(_desc(xs)), _ref(_desc(topk_idx)), _opt(topk_weights),
-                                int(num_experts), _MOE_LAYOUTS[layout], alignment, _ref(_desc(a)), _ref(_desc(a_sf)),
-                                _ref(_desc(gl)), _ref(_desc(pos)), _opt(w), _ref(_desc(ws)), _ffi.stream_of(xq)))
+    _check(_bind.dispatch(xq, xs, topk_idx, topk_weights, int(num_experts), _MOE_LAYOUTS[layout], alignment, a, a_sf, gl,
+                          pos, w, ws, _raw_stream_of(xq)))
     if w is not None and layout == 'masked':
         w = w.view(num_experts, max_m)
     return a, a_sf, gl, pos, w
@@ -537,9 +515,7 @@ def moe_swiglu_apply_weight_to_fp8(x: torch.Tensor, row_weights: Optional[torch.
     else:
         q = torch.empty((m, i2 // 2), dtype=torch.float8_e4m3fn, device=x.device)
         sf = torch.empty((m, i2 // 2 // gran_k), dtype=torch.float32, device=x.device)
-    _check(_lib.dg_moe_swiglu_apply_weight_to_fp8(_ref(_desc(x)), _opt(row_weights), _opt(row_layout),
-                                                  float(clamp_value or 0.0), _ref(_desc(q)), _ref(_desc(sf)),
-                                                  int(gran_k), _ffi.stream_of(x)))
+    _check(_bind.swiglu(x, row_weights, row_layout, float(clamp_value or 0.0), q, sf, int(gran_k), _raw_stream_of(x)))
     return q, sf
 
 
@@ -548,8 +524,7 @@ def moe_combine(y: torch.Tensor, pos: torch.Tensor, topk_weights: Optional[torch
     out[t] = sum over slots of w * y[pos[t, j]] in slot order (w = 1 without
     topk_weights), the one-GPU form of DeepEP's combine."""
     out = torch.empty((pos.shape[0], y.shape[-1]), dtype=torch.bfloat16, device=y.device)
-    _check(_lib.dg_moe_combine(_ref(_desc(y)), _ref(_desc(pos)), _opt(topk_weights), _ref(_desc(out)),
-                               _ffi.stream_of(y)))
+    _check(_bind.combine(y, pos, topk_weights, out, _raw_stream_of(y)))
     return out
 
 
@@ -590,10 +565,8 @@ def m_grouped_fp8_gemm_nt_contiguous_swiglu(a, b, out: Tuple[torch.Tensor, torch
     a_t, sfa = _pair(a, 'a')
     b_t, sfb = _pair(b, 'b')
     q, sf = _pair(out, 'out')
-    _check(_lib.dg_m_grouped_fp8_gemm_nt_contiguous_swiglu(
-        _ref(_desc(a_t)), _ref(_desc(sfa)), _ref(_desc(b_t)), _ref(_desc(sfb)), _ref(_desc(grouped_layout)),
-        _opt(row_weights), float(activation_clamp or 0.0), _ref(_desc(q)), _ref(_desc(sf)),
-        int(bool(use_psum_layout)), int(bool(ensure_zero_padding)), _ffi.stream_of(q)))
+    _check(_bind.contiguous_swiglu(a_t, sfa, b_t, sfb, grouped_layout, row_weights, float(activation_clamp or 0.0), q, sf,
+                                   int(bool(use_psum_layout)), int(bool(ensure_zero_padding)), _raw_stream_of(q)))
 
 
 def m_grouped_fp8_gemm_nt_masked_swiglu(a, b, out: Tuple[torch.Tensor, torch.Tensor], masked_m: torch.Tensor,
@@ -605,10 +578,8 @@ def m_grouped_fp8_gemm_nt_masked_swiglu(a, b, out: Tuple[torch.Tensor, torch.Ten
     a_t, sfa = _pair(a, 'a')
     b_t, sfb = _pair(b, 'b')
     q, sf = _pair(out, 'out')
-    _check(_lib.dg_m_grouped_fp8_gemm_nt_masked_swiglu(
-        _ref(_desc(a_t)), _ref(_desc(sfa)), _ref(_desc(b_t)), _ref(_desc(sfb)), _ref(_desc(masked_m)),
-        int(expected_m), _opt(row_weights), float(activation_clamp or 0.0), _ref(_desc(q)), _ref(_desc(sf)),
-        _ffi.stream_of(q)))
+    _check(_bind.masked_swiglu(a_t, sfa, b_t, sfb, masked_m, int(expected_m), row_weights, float(activation_clamp or 0.0),
+                               q, sf, _raw_stream_of(q)))
 
 
 def per_token_cast_to_fp8_mn_major(x: torch.Tensor, use_ue8m0: bool,
@@ -622,6 +593,5 @@ def per_token_cast_to_fp8_mn_major(x: torch.Tensor, use_ue8m0: bool,
     am = (m + 3) // 4 * 4
     q = torch.empty((m, n), dtype=torch.float8_e4m3fn, device=x.device)
     sf = torch.empty_strided((m, groups), (1, am), dtype=torch.float32, device=x.device)
-    _check(_lib.dg_per_token_cast_to_fp8(_ref(_desc(x)), _ref(_desc(q)), _ref(_desc(sf)), int(gran_k),
-                                         int(bool(use_ue8m0)), _ffi.stream_of(x)))
+    _check(_bind.cast(x, q, sf, int(gran_k), int(bool(use_ue8m0)), _raw_stream_of(x)))
     return q, sf
