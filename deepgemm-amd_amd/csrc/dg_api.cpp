@@ -523,6 +523,30 @@ void launch_1d1d(bool k_grouped, const Fp8GemmArgs& args, hipStream_t stream, in
     launch_fp8_gemm_1d1d_pipe(k_grouped, t, args, stream);
 }
 
+// Workgroup shape of the UE8M0 tiny-M kernel for a dense call, or {256, 256, 2} where
+// the pipelined kernel is faster. Time per round of workgroups on the CUs, measured (us,
+// kb = K blocks; A e4m3, B e2m1): 32 x 32 4.5 + 0.115 kb, 32 x 64 6.5 + 0.19 kb, 64 x 32
+// 4 + 0.285 kb, 64 x 64 4.5 + 0.345 kb, pipelined 256 x 256 6 + 1.15 kb. Measured,
+// pipelined -> the chosen shape: 1 x 7168 x 7168 70 -> 8.6, 48 x 7168 x 7168 70 -> 17,
+// 200 x 7168 x 7168 72 -> 48, 400 x 2112 x 7168 74 -> 26, 48 x 24576 x 1536 21 -> 16,
+// 200 x 7168 x 2048 26 -> 16; it stays pipelined at 100 x 24576 x 1536 (21, 64 x 64 23)
+// and 400 x 7168 x 7168 (73, 79).
+TileConfig choose_ue8m0_tinym(int64_t m, int64_t n, int64_t k, int cus) {
+    struct Shape { int rows, cols; double t0, tk; };
+    static const Shape shapes[] = {{32, 32, 4.5, 0.115}, {32, 64, 6.5, 0.19}, {64, 32, 4.0, 0.285}, {64, 64, 4.5, 0.345}};
+    const double kb = (double)k / 128;
+    // Up to 8 K blocks (pipelined at most 15 us, 6 here) a call keeps the sums in one
+    // chain: the bits of the same call with FP32 scales, which callers compare.
+    if (kb <= 8) return TileConfig{256, 256, 2};
+    double best = (double)ceil_div(ceil_div(m, 256) * ceil_div(n, 256), cus) * (6.0 + 1.15 * kb);
+    TileConfig out{256, 256, 2};
+    for (const auto& s : shapes) {
+        const double cost = (double)ceil_div(ceil_div(m, s.rows) * ceil_div(n, s.cols), cus) * (s.t0 + s.tk * kb);
+        if (cost < best) best = cost, out = TileConfig{s.rows, s.cols, 11};
+    }
+    return out;
+}
+
 bool is_ue8m0_path(const Operands& o, const Recipe& r) {
     const bool fp4 = is_fp4(o.a) || is_fp4(o.b);
     const bool packed = o.sfa.dtype() == DG_I32 || o.sfb.dtype() == DG_I32;
@@ -784,12 +808,23 @@ void run_gemm(GemmKind kind, const Operands& o, const Recipe& r, int64_t m, int6
         args.sfb_gs = grouped_b ? o.sfb.stride(0) : 0;
         args.sfb_row_shift = r.gran_mn_b == 128 ? 7 : 0;
         args.alpha = (ep && ep->kind == DG_EPILOGUE_ALPHA) ? ep->alpha : 1.0f;
-        // The 256 x 256 pipelined kernel takes packed scale words and K % 128 == 0;
-        // everything else runs on the 128 x 128 kernel. A tile override selects
+        // The 256 x 256 pipelined kernel takes packed scale words and K % 128 == 0 (few
+        // rows of it: the tiny-M kernel, variant 11); everything else runs on the 128 x 128 kernel. A tile override selects
         // the kernel by its variant (1: 128 x 128, 2: pipelined).
         const int tv = g_tile_variant.load();
         const bool pipe_ok = fp8_fp4_pipe_supported(args) && grouped_tile_ok(kind, 2, 256, align_m);
         if (tv == 2 && !pipe_ok) DG_UNSUPPORTED("tile override: the pipelined UE8M0 kernel does not take these inputs");
+        if (kind == kNormal && (tv == 0 || tv == 11) && fp8_fp4_tinym_supported(args)) {
+            int cus = 256;
+            try { cus = num_sms_now(); } catch (const Error&) {}
+            TileConfig t = choose_ue8m0_tinym(m, n, k, std::max(1, cus));
+            if (tv == 11) t = {g_tile_m.load(), g_tile_n.load(), 11};
+            if (t.variant == 11) {
+                record_config("fp8_fp4_gemm_ue8m0_tinym", kind, t, m, n, k, groups);
+                launch_fp8_fp4_gemm_tinym(t, args, stream);
+                return;
+            }
+        }
         if (pipe_ok && tv != 1) {
             const TileConfig t{256, 256, 2};
             record_config("fp8_fp4_gemm_ue8m0_pipe", kind, t, m, n, k, groups);
@@ -1691,6 +1726,7 @@ int dg_set_tile_override(int32_t variant, int32_t block_m, int32_t block_n) {
                         : variant == 8 || variant == 9
                             ? ((block_m == 16 || block_m == 32 || block_m == kTinyMRows) &&
                                (block_n == 16 || block_n == 32 || block_n == 64))
+                        : variant == 11 ? ((block_m == 32 || block_m == 64) && (block_n == 32 || block_n == 64))
                         : variant == 10 ? (block_m == 0 && block_n >= 0 && block_n <= 1024)
                                        : (variant == 4 && block_m == 256 && block_n == 256);
         if (!ok) DG_UNSUPPORTED("tile shape not compiled");

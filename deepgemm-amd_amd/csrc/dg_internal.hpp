@@ -98,7 +98,8 @@ struct TileConfig {
     //     most 16 rows on 16 x 16 x 128 MFMAs; block_n = 32 x waves),
     // 6 = 1D1D (block_m 128, block_n = 32 x waves),
     // 8 / 9 = dense tiny M with 8 / 4 waves (block_m 16, block_n 16, 32 or 64
-    //     columns per workgroup: K split over the waves of a workgroup)
+    //     columns per workgroup: K split over the waves of a workgroup),
+    // 11 = UE8M0 tiny M (block_m, block_n 32 or 64)
     int variant = 1;
 };
 
@@ -193,6 +194,11 @@ void launch_fp8_fp4_gemm(GemmKind kind, const TileConfig& cfg, const Fp8Fp4GemmA
 // operands (SFB one row per N row) and K a multiple of 128.
 bool fp8_fp4_pipe_supported(const Fp8Fp4GemmArgs& args);
 void launch_fp8_fp4_gemm_pipe(GemmKind kind, const Fp8Fp4GemmArgs& args, hipStream_t stream);
+// Dense calls of few rows, K split over the waves of a workgroup of block_m x block_n
+// outputs (32 or 64 each; dg_gemm_fp8fp4_tinym.hip): what the pipelined kernel takes,
+// with BF16 D and no C.
+bool fp8_fp4_tinym_supported(const Fp8Fp4GemmArgs& args);
+void launch_fp8_fp4_gemm_tinym(const TileConfig& cfg, const Fp8Fp4GemmArgs& args, hipStream_t stream);
 
 // SF layout kernels.
 struct SfTransposeArgs {

@@ -420,7 +420,8 @@ int32_t dg_get_theoretical_mk_alignment_for_contiguous_layout(int32_t expected_m
  * the 1D1D kernels (7: 128 x 128 or 256 x 256), 8 / 9 = the tiny-M kernel with 8 / 4 waves (block_m = rows
  * per workgroup, 16, 32 or 64; block_n = columns per workgroup, 16, 32 or 64),
  * 10 = the split-K kernel of dg_fp8_fp4_gemm_nt_ws (block_m 0; block_n = K
- * chunks, 0 for the heuristic's count);
+ * chunks, 0 for the heuristic's count), 11 = the UE8M0 tiny-M kernel (block_m and
+ * block_n 32 or 64: rows and columns per workgroup);
  * variant 0 restores the heuristic. Only compiled tile shapes are accepted. */
 int dg_set_tile_override(int32_t variant, int32_t block_m, int32_t block_n);
 

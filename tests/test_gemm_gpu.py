@@ -1522,3 +1522,49 @@ def test_contiguous_block_table(case, shift):
                                                          a[1][r:r + 1].cpu().numpy()),
                                 oquant.dequant_per_block(b[0][ei].view(torch.uint8).cpu().numpy(), b[1][ei].cpu().numpy()))
             assert ogemm.calc_diff(outs[1][r:r + 1].view(torch.bfloat16).float().cpu().numpy(), ref) < 1e-3
+
+
+@pytest.mark.parametrize('m,n,k', [(1, 32, 128), (33, 72, 896), (64, 2112, 1152), (100, 264, 7168), (130, 520, 128 * 9)])
+@pytest.mark.parametrize('b_fp4,gka,gkb', [(True, 128, 32), (True, 32, 32), (False, 128, 128), (False, 32, 128)])
+def test_ue8m0_tiny_m(m, n, k, b_fp4, gka, gkb):
+    """Every workgroup shape of the UE8M0 tiny-M kernel (ragged rows and columns, fewer K
+    blocks than waves, uneven shares of them) against the FP64 oracle: one BF16 ulp plus
+    2^-15 sum |a b|; shapes agree bit for bit (an output's K split does not depend on
+    them), reruns too, and alpha scales the sum before the rounding."""
+    a_np, b_np = gen.randn_bf16((m, k), m + k), gen.randn_bf16((n, k), n)
+    qa, sfa = oquant.per_token_cast_to_fp8(a_np, use_ue8m0=True, gran_k=gka)
+    if b_fp4:
+        qb, sfb = oquant.per_token_cast_to_fp4(b_np, use_ue8m0=True, gran_k=gkb)
+        b_deq = oquant.dequant_fp4(qb, sfb, gkb)
+    else:
+        qb, sfb = oquant.per_token_cast_to_fp8(b_np, use_ue8m0=True, gran_k=gkb)
+        b_deq = oquant.dequant_per_token(qb, sfb, gran_k=gkb)
+    a_deq = oquant.dequant_per_token(qa, sfa, gran_k=gka)
+    ref = ogemm.gemm_nt(a_deq, b_deq)
+    tol = np.abs(ref) * 2.0 ** -8 + 2.0 ** -15 * ogemm.gemm_nt(np.abs(a_deq), np.abs(b_deq))
+    a = (e4m3(qa), deep_gemm.get_mn_major_tma_aligned_packed_ue8m0_tensor(f32(sfa)))
+    b = (gen.to_dev(qb, torch.int8 if b_fp4 else torch.float8_e4m3fn),
+         deep_gemm.get_mn_major_tma_aligned_packed_ue8m0_tensor(f32(sfb)))
+    outs = []
+    for rows in (32, 64):
+        for cols in (32, 64):
+            for _ in range(2):
+                d = sentinel_bf16((m, n))
+                deep_gemm.set_tile_override(rows, cols, variant=11)
+                try:
+                    deep_gemm.fp8_fp4_gemm_nt(a, b, d, recipe_a=(1, gka), recipe_b=(1, gkb))
+                finally:
+                    deep_gemm.set_tile_override(0, 0)
+                assert f'tinym v11 kind=normal block_m={rows} block_n={cols}' in deep_gemm.get_last_config()
+                outs.append(d)
+    torch.cuda.synchronize()
+    assert np.all(np.abs(outs[0].float().cpu().numpy() - ref) <= tol)
+    for o in outs[1:]:
+        assert torch.equal(o.view(torch.int16), outs[0].view(torch.int16))
+    d = sentinel_bf16((m, n))
+    deep_gemm.set_tile_override(32, 32, variant=11)
+    try:
+        deep_gemm.fp8_fp4_gemm_nt(a, b, d, recipe_a=(1, gka), recipe_b=(1, gkb), alpha=0.5)
+    finally:
+        deep_gemm.set_tile_override(0, 0)
+    assert torch.equal(d.float(), (outs[0].float() * 0.5).bfloat16().float())   # (a power of two: exact)
