@@ -47,6 +47,16 @@ constexpr int kDenseStreamRows = 64;
 constexpr int64_t kTinyMWideMaxK = 8192;
 constexpr int64_t kTinyMWideMaxTiles = 64;   // 128 x 128 tiles of the tiled launch
 constexpr int kTinyMStreamGrid = 64;
+// Dense calls whose tiles come out as 128 x 128 take the kernel that splits K blocks over
+// two wave groups up to three quarters of a round of tiles, with K from 2048 and B of at
+// most 32 MB: 19-25% faster there with the weights in cache (the figures are beside the
+// kernel), even to 6% with weights from HBM. Beyond, HBM latency shows, as it keeps fewer stages
+// in flight (weights from HBM, pipelined -> split): 1024 x 4096 x 7168 (a full round)
+// 42.4 -> 44.1 us, 256 x 7168 x 7168 (51 MB) 41.5 -> 44.7; K = 1536 and less is even or
+// gains under 1 us; a partial last K block lost 5% (2000 x 1536 x 3008), so it has no
+// schedule for one.
+constexpr int64_t kKsplitMinK = 2048;
+constexpr int64_t kKsplitMaxWeight = (int64_t)32 << 20;   // B bytes
 
 int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
@@ -649,6 +659,13 @@ void run_gemm(GemmKind kind, const Operands& o, const Recipe& r, int64_t m, int6
             DG_UNSUPPORTED("tile override: the split-K kernel runs dense calls of at most 64 rows with K % 128 == 0, "
                            "BF16 D and no C");
         }
+        if (tv == 12) {
+            if (kind != kNormal || !fp8_ksplit_supported(args))
+                DG_UNSUPPORTED("tile override: the K-split kernel runs dense calls with K % 128 == 0, BF16 D and no C");
+            record_config("fp8_gemm_1d2d", kind, TileConfig{128, 128, 12}, m, n, k, groups);
+            launch_fp8_gemm_ksplit(args, stream);
+            return;
+        }
         TileConfig t;
         // Dense calls of at most kDenseStreamRows rows are weight-stream bound: they
         // run on the streaming kernel as one group (layout null), which loads only
@@ -712,6 +729,14 @@ void run_gemm(GemmKind kind, const Operands& o, const Recipe& r, int64_t m, int6
             if (tv == 0 && is_persistent_route(kind, t, args, m_rows, n, k)) t.variant = 4;
             if (tv == 0 && kind == kContiguous && is_table_route(m_rows, n, k, groups, args.grid_limit, align_m))
                 t = {256, 256, 4};
+            if (tv == 0 && kind == kNormal && t.variant == 2 && t.block_m == 128 && t.block_n == 128 && k >= kKsplitMinK &&
+                n * k <= kKsplitMaxWeight && 4 * ceil_div(m_rows, 128) * ceil_div(n, 128) <= 3 * args.grid_limit &&
+                fp8_ksplit_supported(args)) {
+                t.variant = 12;
+                record_config("fp8_gemm_1d2d", kind, t, m, n, k, groups);
+                launch_fp8_gemm_ksplit(args, stream);
+                return;
+            }
         }
         if (!grouped_tile_ok(kind, t.variant, t.block_m, align_m))
             DG_UNSUPPORTED("M alignment for contiguous layout must be a multiple of 64");
@@ -1726,6 +1751,7 @@ int dg_set_tile_override(int32_t variant, int32_t block_m, int32_t block_n) {
                         : variant == 8 || variant == 9
                             ? ((block_m == 16 || block_m == 32 || block_m == kTinyMRows) &&
                                (block_n == 16 || block_n == 32 || block_n == 64))
+                        : variant == 12 ? (block_m == 128 && block_n == 128)
                         : variant == 11 ? ((block_m == 32 || block_m == 64) && (block_n == 32 || block_n == 64))
                         : variant == 10 ? (block_m == 0 && block_n >= 0 && block_n <= 1024)
                                        : (variant == 4 && block_m == 256 && block_n == 256);

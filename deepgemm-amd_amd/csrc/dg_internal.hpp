@@ -99,7 +99,8 @@ struct TileConfig {
     // 6 = 1D1D (block_m 128, block_n = 32 x waves),
     // 8 / 9 = dense tiny M with 8 / 4 waves (block_m 16, block_n 16, 32 or 64
     //     columns per workgroup: K split over the waves of a workgroup),
-    // 11 = UE8M0 tiny M (block_m, block_n 32 or 64)
+    // 11 = UE8M0 tiny M (block_m, block_n 32 or 64),
+    // 12 = dense, K blocks split over two wave groups (128 x 128)
     int variant = 1;
 };
 
@@ -143,6 +144,11 @@ bool fp8_1d2d_tile_supported(int block_m, int block_n);
 void launch_fp8_gemm_1d2d_v2(GemmKind kind, const TileConfig& cfg, const Fp8GemmArgs& args,
                              hipStream_t stream);
 bool fp8_1d2d_v2_tile_supported(int block_m, int block_n);
+
+// Dense calls of at most a round of 128 x 128 tiles, even and odd K blocks on two
+// groups of waves (dg_gemm_fp8_ksplit.hip): BF16 D without C, K a multiple of 16.
+bool fp8_ksplit_supported(const Fp8GemmArgs& args);
+void launch_fp8_gemm_ksplit(const Fp8GemmArgs& args, hipStream_t stream);
 
 // The masked weight-streaming kernel (dg_gemm_fp8_masked.hip): K a multiple of
 // 128 (at most 128 blocks), BF16 D without C. `waves` = block_n / 32, 4 to 8.

@@ -31,7 +31,7 @@ import os
 import sys
 
 GEMM_KEYS = ('fp8_gemm_1d2d', 'fp8_fp4_gemm', 'fp8_gemm_1d2d_pipe', 'fp8_gemm_masked_stream', 'fp8_gemm_1d1d',
-             'fp8_gemm_tinym', 'fp8_gemm_splitk', 'moe_swiglu_cast_kernel')
+             'fp8_gemm_tinym', 'fp8_gemm_splitk', 'fp8_gemm_ksplit', 'moe_swiglu_cast_kernel')
 CAST_KEYS = ('per_token_cast_kernel',)   # the cast workload's kernel (GEMM workloads also cast while setting up)
 MOE_DISPATCH_KEYS = ('moe_count_kernel', 'moe_scan_kernel', 'moe_starts_kernel', 'moe_scatter_kernel')
 COPY_KEY = 'neg_kernel'

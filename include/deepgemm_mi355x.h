@@ -421,7 +421,8 @@ int32_t dg_get_theoretical_mk_alignment_for_contiguous_layout(int32_t expected_m
  * per workgroup, 16, 32 or 64; block_n = columns per workgroup, 16, 32 or 64),
  * 10 = the split-K kernel of dg_fp8_fp4_gemm_nt_ws (block_m 0; block_n = K
  * chunks, 0 for the heuristic's count), 11 = the UE8M0 tiny-M kernel (block_m and
- * block_n 32 or 64: rows and columns per workgroup);
+ * block_n 32 or 64: rows and columns per workgroup), 12 = the K-split kernel of
+ * dense calls (128 x 128);
  * variant 0 restores the heuristic. Only compiled tile shapes are accepted. */
 int dg_set_tile_override(int32_t variant, int32_t block_m, int32_t block_n);
 

@@ -1568,3 +1568,41 @@ def test_ue8m0_tiny_m(m, n, k, b_fp4, gka, gkb):
     finally:
         deep_gemm.set_tile_override(0, 0)
     assert torch.equal(d.float(), (outs[0].float() * 0.5).bfloat16().float())   # (a power of two: exact)
+
+
+@pytest.mark.parametrize('m,n,k', [
+    (1, 8, 128),           # one row, a short tile and one block: the odd group has none
+    (128, 128, 128),
+    (129, 136, 256),       # a row and eight columns past a tile, a block per group
+    (100, 200, 384),       # the odd group's last block is missing
+    (257, 264, 1024),      # scales four blocks at a time where K-major
+    (1100, 104, 1152),     # more m-blocks than a raster group; an odd number of blocks
+    (517, 384, 7168),
+])
+@pytest.mark.parametrize('row_major_sfa', [False, True])
+def test_dense_k_split_groups(m, n, k, row_major_sfa):
+    """Even and odd K blocks on two wave groups, against the FP64 oracle: one BF16 ulp plus
+    2^-15 sum |a b|; what lies past K in memory, NaN included, stays out of the sums."""
+    a_np, b_np = gen.randn_bf16((m, k), m + k), gen.randn_bf16((n, k), n)
+    qa, sfa = oquant.per_token_cast_to_fp8(a_np, use_ue8m0=False, gran_k=128)
+    qb, sfb = oquant.per_block_cast_to_fp8(b_np, use_ue8m0=False)
+    a_deq, b_deq = oquant.dequant_per_token(qa, sfa, gran_k=128), oquant.dequant_per_block(qb, sfb)
+    ref = ogemm.gemm_nt(a_deq, b_deq)
+    tol = np.abs(ref) * 2.0 ** -8 + 2.0 ** -15 * ogemm.gemm_nt(np.abs(a_deq), np.abs(b_deq))
+    sf = f32(sfa) if row_major_sfa else deep_gemm.get_mn_major_tma_aligned_tensor(f32(sfa))
+    outs = []
+    for pad in (0, 128):   # rows of K bytes, and rows followed by NaN
+        a, b = [torch.full((r, k + pad), 0x7F, dtype=torch.uint8, device='cuda').view(torch.float8_e4m3fn) for r in (m, n)]
+        a.view(torch.uint8)[:, :k] = e4m3(qa).view(torch.uint8)
+        b.view(torch.uint8)[:, :k] = e4m3(qb).view(torch.uint8)
+        d = sentinel_bf16((m, n))
+        deep_gemm.set_tile_override(128, 128, variant=12)
+        try:
+            deep_gemm.fp8_gemm_nt((a[:, :k], sf), (b[:, :k], f32(sfb)), d)
+        finally:
+            deep_gemm.set_tile_override(0, 0)
+        assert 'v12 kind=normal block_m=128 block_n=128' in deep_gemm.get_last_config()
+        outs.append(d)
+    torch.cuda.synchronize()
+    assert np.all(np.abs(outs[0].float().cpu().numpy() - ref) <= tol)
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
