@@ -316,10 +316,12 @@ bool grouped_tile_ok(GemmKind kind, int variant, int bm, int align_m) {
     return true;
 }
 
-TileConfig choose_tile_1d2d(GemmKind kind, int64_t m_rows, int64_t n, int64_t k, int64_t groups, int align_m) {
+// offsets_fit: the operands' row pitches fit the pipelined kernel (fp8_pipe_offsets_fit).
+TileConfig choose_tile_1d2d(GemmKind kind, int64_t m_rows, int64_t n, int64_t k, int64_t groups, int align_m,
+                            bool offsets_fit) {
     const int tv = g_tile_variant.load(), tm = g_tile_m.load(), tn = g_tile_n.load();
     // The pipelined kernel keeps one SFB value per K block in LDS (up to 1024 blocks).
-    const bool pipe_ok = ceil_div(k, 128) <= 1024;
+    const bool pipe_ok = offsets_fit && ceil_div(k, 128) <= 1024;
     // K % 128 != 0: the 256 x 256 pipelined tile is built for dense launches only,
     // and an override takes it with whole K blocks only (the other tiles give the
     // same bits).
@@ -708,7 +710,9 @@ void run_gemm(GemmKind kind, const Operands& o, const Recipe& r, int64_t m, int6
             t = {rows_hint <= kStream16Rows ? kStream16Rows : kMaskedStreamRows,
                  32 * fp8_masked_stream_waves(n, groups, args.grid_limit), 5};
         } else {
-            t = choose_tile_1d2d(kind, m_rows, n, k, kind == kMasked ? groups : 1, align_m);
+            // (a wider pitch than the pipelined kernel's offsets hold: the register-staged one)
+            const bool offsets_fit = fp8_pipe_offsets_fit(args);
+            t = choose_tile_1d2d(kind, m_rows, n, k, kind == kMasked ? groups : 1, align_m, offsets_fit);
             // Masked groups far below max_m: one workgroup per tile launches every
             // m-block of max_m, and each empty workgroup still holds a CU's LDS while
             // it starts and exits; the persistent walk visits only the m-blocks below
@@ -727,7 +731,7 @@ void run_gemm(GemmKind kind, const Operands& o, const Recipe& r, int64_t m, int6
             // rounds) and keep the per-tile launch and its column split; at 1-3.5
             // rounds it loses (4096 x 7168 x 2048 +5%), and with FP32 C it is even.
             if (tv == 0 && is_persistent_route(kind, t, args, m_rows, n, k)) t.variant = 4;
-            if (tv == 0 && kind == kContiguous && is_table_route(m_rows, n, k, groups, args.grid_limit, align_m))
+            if (tv == 0 && kind == kContiguous && offsets_fit && is_table_route(m_rows, n, k, groups, args.grid_limit, align_m))
                 t = {256, 256, 4};
             if (tv == 0 && kind == kNormal && t.variant == 2 && t.block_m == 128 && t.block_n == 128 && k >= kKsplitMinK &&
                 n * k <= kKsplitMaxWeight && 4 * ceil_div(m_rows, 128) * ceil_div(n, 128) <= 3 * args.grid_limit &&
@@ -1456,10 +1460,10 @@ void k_grouped_impl(const dg_tensor* a_, const dg_tensor* sfa_, const dg_tensor*
     DG_CHECK(numel(gl) == g);
     DG_CHECK(gl.on_device());
     DG_CHECK((int64_t)num_ks == g);
-    int64_t sum_k = 0;
+    int64_t sum_k = 0, max_k = 0;
     for (int32_t i = 0; i < num_ks; ++i) {
         DG_CHECK(ks[i] >= 0 && ks[i] % 128 == 0);
-        sum_k += ks[i];
+        sum_k += ks[i], max_k = std::max<int64_t>(max_k, ks[i]);
     }
     DG_CHECK(numel(a) == sum_k * m);
     DG_CHECK(numel(b) == sum_k * n);
@@ -1501,6 +1505,7 @@ void k_grouped_impl(const dg_tensor* a_, const dg_tensor* sfa_, const dg_tensor*
     args.m = (int32_t)m, args.n = (int32_t)n, args.k = 0;
     args.num_groups = (int32_t)g;
     args.out_f32 = 1;
+    args.lda = args.ldb = max_k;   // (the widest group's pitch; the kernels take each group's from ks)
     args.ldd = n, args.ldc = n, args.d_gs = m * n, args.c_gs = m * n;
     args.sfa_sm = sfa.stride(0), args.sfa_sk = sfa.stride(1);
     args.sfb_sn = sfb.stride(0), args.sfb_sk = sfb.stride(1);

@@ -243,6 +243,9 @@ void launch_nw(const Fp8GemmArgs& a, hipStream_t stream) {
 
 void launch_fp8_gemm_1d1d(bool k_grouped, int waves, const Fp8GemmArgs& a, hipStream_t stream) {
     DG_CHECK(a.out_f32 && a.c != nullptr && a.k % kBK == 0);
+    if (!lane_offsets_fit(std::min(a.m, 128), std::max(a.lda, a.sfa_sm * 4)) ||
+        !lane_offsets_fit(std::min(a.n, 256), std::max(a.ldb, a.sfb_sn * 4)))
+        DG_UNSUPPORTED("the row pitch of an operand is too wide for the streaming 1D1D kernel");
     switch (waves * 2 + (k_grouped ? 1 : 0)) {
         case 8: launch_nw<4, 0>(a, stream); break;
         case 9: launch_nw<4, 1>(a, stream); break;

@@ -106,7 +106,7 @@ fp8_gemm_ksplit_kernel(const Fp8GemmArgs p, const int num_m_blocks, const int nu
     constexpr int kLoads = KSA ? 8 : 9;   // per wave and stage
     auto issue = [&](int pr) {
         if (KSA && (pr & 1) == 0) issue_sfa(pr >> 1);   // (before the stage's own: the waits below cover it)
-                const int kb = min(2 * pr + kg, num_kb - 1);
+        const int kb = min(2 * pr + kg, num_kb - 1);
         const uint32_t lds = smem_lds + (pr & 1) * kStageBytes + kg * kBlockBytes;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -246,7 +246,8 @@ fp8_gemm_ksplit_kernel(const Fp8GemmArgs p, const int num_m_blocks, const int nu
 
 bool fp8_ksplit_supported(const Fp8GemmArgs& a) {
     return a.m > 0 && a.n > 0 && a.k > 0 && a.k % kBK == 0 && a.k <= kMaxKBlocks * kBK && !a.out_f32 && a.c == nullptr && a.num_groups == 1 &&
-           a.layout == nullptr && a.lda < (1 << 24) && a.ldb < (1 << 24) && a.sfa_sm < (1 << 20);  // 32-bit lane offsets
+           a.layout == nullptr && lane_offsets_fit(std::min(a.m, kTile), std::max(a.lda, a.sfa_sm * 4)) &&
+           lane_offsets_fit(std::min(a.n, kTile), a.ldb);
 }
 
 void launch_fp8_gemm_ksplit(const Fp8GemmArgs& a, hipStream_t stream) {

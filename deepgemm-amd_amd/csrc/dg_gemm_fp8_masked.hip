@@ -45,6 +45,8 @@
 // blocks, BF16 D without C, 16-byte aligned A/B/D rows.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "dg_internal.hpp"
 #include "dg_kernel_common.hpp"
 #include "dg_epilogue.hpp"
@@ -575,7 +577,9 @@ void launch_nw(const Fp8GemmArgs& a, int mfma16, hipStream_t stream) {
 }  // namespace
 
 bool fp8_masked_stream_supported(const Fp8GemmArgs& a) {
-    return a.k > 0 && a.k % kBK == 0 && a.k / kBK <= kMaxKB && !a.out_f32 && a.c == nullptr && a.n > 0;
+    return a.k > 0 && a.k % kBK == 0 && a.k / kBK <= kMaxKB && !a.out_f32 && a.c == nullptr && a.n > 0 &&
+           lane_offsets_fit(std::min(a.m, kMaskedStreamRows), std::max(a.lda, a.sfa_sm * 4)) &&
+           lane_offsets_fit(std::min(a.n, 256), a.ldb);
 }
 
 int fp8_masked_stream_waves(int64_t n, int64_t groups, int cus) {

@@ -364,20 +364,28 @@ fp8_gemm_1d2d_pipe_kernel(const Fp8GemmArgs p_arg, const int num_m_blocks, const
     // hoisting the offsets into registers held across the loop, and a branch in
     // the middle of the MFMA sequence would cost registers too.
     const uint32_t chunk_off = (pc ^ swz_g((wave & 1) * 8 + rs)) << 4;
-    const int sa_row = wave * SA_ROWS_PER_WAVE + lane;
-    const uint32_t voff_sa = (uint32_t)(min(sa_row, a_rows - 1) * p.sfa_sm) * 4u;
+    // The wave's SFA rows from row sa_r0 (its first, or the last valid one). All lane
+    // offsets are 32-bit, from a wave-uniform 64-bit base at the wave's own rows:
+    // they hold the pitch of 8 rows of A or B and of at most 64 of the scales, which the
+    // host checks (fp8_pipe_offsets_fit).
+    const int sa_r0 = min(wave * SA_ROWS_PER_WAVE, a_rows - 1);
+    const float* __restrict__ sa_wave = sa_base + (int64_t)sa_r0 * p.sfa_sm;
+    const uint32_t voff_sa = (uint32_t)(min(min(lane, SA_ROWS_PER_WAVE - 1), a_rows - 1 - sa_r0) * p.sfa_sm) * 4u;
     const int sb_seg = min(wave, SB_SEGS - 1);   // SB1D: surplus waves repeat the last segment
     // SB1D: the column (of 32) whose scale this lane holds
     const int sb_lane = ((lane >> 2) & 3) * 8 + lhalf * 4 + (lane & 3);
-    const uint32_t voff_sb = SB1D ? (uint32_t)(min(sb_seg * 64 + lane, b_rows - 1) * p.sfb_sn) * 4u : 0u;
+    const int sb_r0 = min(sb_seg * 64, b_rows - 1);
+    const float* __restrict__ sb_wave = sb_base + (int64_t)sb_r0 * p.sfb_sn;
+    const uint32_t voff_sb = SB1D ? (uint32_t)(min(lane, b_rows - 1 - sb_r0) * p.sfb_sn) * 4u : 0u;
     // Load of segment seg (8 rows): the segment's first row goes into the
     // wave-uniform SGPR base (clamped to the last valid row), and the lane adds its
     // own row and chunk, vlane = rs * ld + chunk_off, a loop-invariant register.
     // Lanes past the last valid row are clamped by one v_min_u32 against a uniform
     // limit, the last valid row's final chunk: they load bytes of that row, which
-    // only feed outputs past the edge (never stored). The limit is laundered so the
-    // per-segment minimum is recomputed at each issue instead of being held in a
-    // register across the loop.
+    // only feed outputs past the edge (never stored). It counts a segment's rows (at
+    // most 7 past the first), not the tile's: 255 rows of a wide pitch pass 32 bits.
+    // The limit is laundered so the per-segment minimum is recomputed at each issue
+    // instead of being held in a register across the loop.
     const uint32_t vlane_a = (uint32_t)rs * (uint32_t)lda + chunk_off;
     const uint32_t vlane_b = (uint32_t)rs * (uint32_t)ldb + chunk_off;
     // last_chunk: the offset of the K block's last chunk (the partial block of a K
@@ -387,7 +395,7 @@ fp8_gemm_1d2d_pipe_kernel(const Fp8GemmArgs p_arg, const int num_m_blocks, const
     auto seg_load = [&](const uint8_t* kb_base, int seg, int rows, int64_t ld, uint32_t vlane, uint32_t lds,
                         uint32_t last_chunk = kBK - 16) {
         const int rb = min(seg * 8, rows - 1);
-        uint32_t lim = (uint32_t)(rows - 1 - rb) * (uint32_t)ld + last_chunk;
+        uint32_t lim = (uint32_t)min(rows - 1 - rb, 7) * (uint32_t)ld + last_chunk;
         asm volatile("" : "+s"(lim));
         dma16_saddr(kb_base + (int64_t)rb * ld, min(vlane, lim), lds);
     };
@@ -412,7 +420,7 @@ fp8_gemm_1d2d_pipe_kernel(const Fp8GemmArgs p_arg, const int num_m_blocks, const
     const uint32_t vlane_sag = (uint32_t)(lane / KSA_LPR) * sag_row_bytes + (lane % KSA_LPR) * 16u;
     auto issue_segment = [&](int g, int j, bool whole) {
         const int rb = min(j * KSA_RPS, a_rows - 1);
-        uint32_t lim = (uint32_t)(a_rows - 1 - rb) * sag_row_bytes + (KSA_LPR - 1) * 16u;
+        uint32_t lim = (uint32_t)min(a_rows - 1 - rb, KSA_RPS - 1) * sag_row_bytes + (KSA_LPR - 1) * 16u;
         asm volatile("" : "+s"(lim));
         dma16_saddr_masked(whole ? __builtin_amdgcn_read_exec() : seg_exec,
                            reinterpret_cast<const uint8_t*>(sa_base + KSA * g + (int64_t)rb * p.sfa_sm),
@@ -446,11 +454,11 @@ fp8_gemm_1d2d_pipe_kernel(const Fp8GemmArgs p_arg, const int num_m_blocks, const
         }
         if constexpr (!KSA)
             if (part != 2)
-                dma4_saddr(reinterpret_cast<const uint8_t*>(sa_base + (int64_t)kb * p.sfa_sk), voff_sa,
+                dma4_saddr(reinterpret_cast<const uint8_t*>(sa_wave + (int64_t)kb * p.sfa_sk), voff_sa,
                            stage_lds + SA_OFF + wave * 256);
         if constexpr (SB1D)   // (with the A side: block kb's scales are read after its B side is refilled)
             if (part != 2)
-                dma4_saddr(reinterpret_cast<const uint8_t*>(sb_base + (int64_t)kb * p.sfb_sk), voff_sb,
+                dma4_saddr(reinterpret_cast<const uint8_t*>(sb_wave + (int64_t)kb * p.sfb_sk), voff_sb,
                            stage_lds + SB_OFF + sb_seg * 256);
     };
 
@@ -807,7 +815,9 @@ fp8_gemm_1d2d_pipe_kernel(const Fp8GemmArgs p_arg, const int num_m_blocks, const
                     const int seg = i * NW + wave;
                     seg_load(b2, seg, b_rows2, ldb, vlane_b, smem_lds + BM * kBK + seg * 1024);
                 }
-                dma4_saddr(reinterpret_cast<const uint8_t*>(sa2), (uint32_t)(min(sa_row, a_rows2 - 1) * p.sfa_sm) * 4u,
+                const int sa2_r0 = min(wave * SA_ROWS_PER_WAVE, a_rows2 - 1);
+                dma4_saddr(reinterpret_cast<const uint8_t*>(sa2 + (int64_t)sa2_r0 * p.sfa_sm),
+                           (uint32_t)(min(min(lane, SA_ROWS_PER_WAVE - 1), a_rows2 - 1 - sa2_r0) * p.sfa_sm) * 4u,
                            smem_lds + SA_OFF + wave * 256);
                 pf_issued = true;
             };
@@ -853,6 +863,7 @@ void launch_kind(const Fp8GemmArgs& a, hipStream_t stream) {
     if (grid == 0) return;
     DG_CHECK(grid < (int64_t)1 << 31);
     DG_CHECK((a.k + kBK - 1) / kBK <= kMaxKBlocks);
+    if (!fp8_pipe_offsets_fit(a)) DG_UNSUPPORTED("the row pitch of an operand is too wide for the pipelined kernel");
     if (PERSIST && KIND == kContiguous)   // (the block table holds up to one tile per 128 rows)
         grid = (int64_t)((a.m + 127) / 128) * num_n_blocks;
     if (PERSIST) grid = std::min<int64_t>(grid, std::max(1, a.grid_limit));
@@ -945,6 +956,8 @@ void launch_1d1d_kind(const Fp8GemmArgs& a, hipStream_t stream) {
     if (grid == 0) return;
     DG_CHECK(grid < (int64_t)1 << 31);
     DG_CHECK(a.out_f32 && a.c != nullptr && a.k % kBK == 0);
+    if (!fp8_pipe_offsets_fit(a) || !lane_offsets_fit(std::min(a.n, 64), a.sfb_sn * 4))
+        DG_UNSUPPORTED("the row pitch of an operand is too wide for the 1D1D kernel");
     const int raster_gm = choose_raster_gm(BM, BN, num_m_blocks);
     hipLaunchKernelGGL((fp8_gemm_1d2d_pipe_kernel<BM, BN, WGM, WGN, 2, KIND, 1, 1, 0, 0, 1>), dim3((unsigned)grid),
                        dim3(WGM * WGN * 64), 0, stream, a, num_m_blocks, num_n_blocks, raster_gm);

@@ -33,6 +33,8 @@
 // without C, 16-byte aligned A and B rows.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "dg_internal.hpp"
 #include "dg_kernel_common.hpp"
 #include "dg_lds_dma.hpp"
@@ -229,7 +231,9 @@ void launch_rt(const Fp8GemmArgs& a, const SplitKPlan& pl, float* ws, hipStream_
 
 bool fp8_splitk_supported(const Fp8GemmArgs& a) {
     return a.m > 0 && a.m <= kSplitKMaxRows && a.n > 0 && a.k > 0 && a.k % kBK == 0 && !a.out_f32 &&
-           a.c == nullptr && a.num_groups == 1 && a.layout == nullptr;
+           a.c == nullptr && a.num_groups == 1 && a.layout == nullptr &&
+           lane_offsets_fit(std::min(a.m, 8), a.lda) && lane_offsets_fit(std::min(a.n, 8), a.ldb) &&
+           lane_offsets_fit(a.m, a.sfa_sm * 4) && lane_offsets_fit(std::min(a.k / kBK, kSplitKMaxChunk), a.sfb_sk * 4);
 }
 
 SplitKPlan plan_fp8_splitk(int64_t m, int64_t n, int64_t k, int cus, int splits) {

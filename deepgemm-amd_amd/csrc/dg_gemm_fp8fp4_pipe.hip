@@ -19,6 +19,7 @@
 // the 128 x 128 kernel (dg_gemm_fp8fp4.hip).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "dg_internal.hpp"
@@ -413,7 +414,8 @@ void launch_kind(const Fp8Fp4GemmArgs& a, hipStream_t stream) {
 bool fp8_fp4_pipe_supported(const Fp8Fp4GemmArgs& a) {
     return a.sfa_packed && a.sfb_packed && a.sfa_sm == 1 && a.sfb_sn == 1 && a.sfb_row_shift == 0 &&
            a.k > 0 && a.k % kBK == 0 && (a.gran_k_a == 32 || a.gran_k_a == 128) &&
-           (a.gran_k_b == 32 || a.gran_k_b == 128);
+           (a.gran_k_b == 32 || a.gran_k_b == 128) && lane_offsets_fit(std::min(a.m, 256), a.lda) &&
+           lane_offsets_fit(std::min(a.n, 256), a.ldb);
 }
 
 void launch_fp8_fp4_gemm_pipe(GemmKind kind, const Fp8Fp4GemmArgs& args, hipStream_t stream) {

@@ -90,6 +90,17 @@ struct Fp8GemmArgs {
     float sw_clamp;                    // <= 0: no clamp
 };
 
+// Whether the offsets of `rows` rows of `pitch` bytes from the first, and the 128 bytes
+// that a row's loads reach, fit the unsigned 32-bit lane offsets of the kernels' LDS loads.
+inline bool lane_offsets_fit(int64_t rows, int64_t pitch) {
+    return rows <= 1 || pitch <= (((int64_t)1 << 32) - 128) / (rows - 1);
+}
+// The pipelined kernel's: segments of 8 rows of A and B, and of at most 64 rows of SFA.
+inline bool fp8_pipe_offsets_fit(const Fp8GemmArgs& a) {
+    return lane_offsets_fit(a.m < 8 ? a.m : 8, a.lda) && lane_offsets_fit(a.n < 8 ? a.n : 8, a.ldb) &&
+           lane_offsets_fit(a.m < 64 ? a.m : 64, a.sfa_sm * 4);
+}
+
 struct TileConfig {
     int block_m;
     int block_n;
