@@ -224,7 +224,9 @@ void launch_fmt(const Fp8Fp4GemmArgs& a, int rows, int cols, hipStream_t stream)
 }  // namespace
 
 bool fp8_fp4_tinym_supported(const Fp8Fp4GemmArgs& a) {
-    return fp8_fp4_pipe_supported(a) && !a.a_fp4 && a.layout == nullptr && a.num_groups == 1 && !a.out_f32 && a.c == nullptr;
+    // (row groups on the grid's y axis)
+    return fp8_fp4_pipe_supported(a) && !a.a_fp4 && a.layout == nullptr && a.num_groups == 1 && !a.out_f32 &&
+           a.c == nullptr && a.m <= 65535 * 32;
 }
 
 void launch_fp8_fp4_gemm_tinym(const TileConfig& cfg, const Fp8Fp4GemmArgs& args, hipStream_t stream) {

@@ -399,3 +399,16 @@ def test_epilogue_python_resolution():
         deep_gemm.k_grouped_fp8_gemm_nt_contiguous(a, b, d, [128], torch.zeros(1, dtype=torch.int32),
                                                    epilogue=ep.Identity())
     assert isinstance(ep.Alpha(0.5), ep.Epilogue) and ep.Alpha(0.5).alpha == 0.5
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason='the accepted call would launch on fake addresses')
+@pytest.mark.parametrize('m,kernel', [(65535 * 32, 'tinym'), (65535 * 32 + 1, 'pipe')])
+def test_ue8m0_row_groups_fit_the_grid(m, kernel):
+    """Narrow outputs of very many rows: the tiny-M kernel up to the row groups that its
+    grid holds, the pipelined one beyond (never refused for the grid)."""
+    n, k = 32, 32768
+    st, msg = call_nt(fake((m, k), _ffi.DG_E4M3), fake((m, k // 512), _ffi.DG_I32, strides=(1, (m + 3) // 4 * 4)),
+                      fake((n, k), _ffi.DG_E4M3, addr=0x20000000), fake((n, k // 512), _ffi.DG_I32, strides=(1, n)),
+                      fake((m, n), _ffi.DG_BF16), recipe=_ffi.recipe_struct(None, (1, 128), (1, 128)))
+    assert st == _ffi.DG_ERR_HIP, msg   # (only for want of a device)
+    assert f'ue8m0_{kernel} ' in deep_gemm.get_last_config()
