@@ -112,6 +112,22 @@ T* pointer(PyObject* o) {
     return static_cast<T*>(p);
 }
 
+// Runs f without the GIL: a launch blocks while the stream's queue is full (or its module
+// loads), an allocation while the device synchronizes, and the other threads run
+// meanwhile, as through ctypes. f sees plain values and C++ tensors only.
+template <typename F>
+auto unlocked(F&& f) {
+    struct Released {
+        PyThreadState* state = PyEval_SaveThread();
+        ~Released() { PyEval_RestoreThread(state); }
+    } released;
+    return f();
+}
+template <typename E, typename... A>
+int32_t call(E entry, A... args) {
+    return unlocked([&] { return entry(args...); });
+}
+
 // Runs f with exceptions turned into Python's: nothing leaves these functions.
 template <typename F>
 PyObject* guarded(Py_ssize_t nargs, Py_ssize_t want, F&& f) {
@@ -159,14 +175,16 @@ PyObject* gemm_nt(PyObject*, PyObject* const* a, Py_ssize_t n) {
         if (!c.given && ta.d.ndim == 2 && tb.d.ndim > 0 && ta.d.sizes[0] <= 64 && d.d.dtype == DG_BF16) {
             const int64_t bytes = g_entry.workspace_size(ta.d.sizes[0], tb.d.sizes[0], ta.d.sizes[1]);
             if (bytes > 0) {
-                const at::Tensor ws = at::empty({bytes}, tensor(a[4]).options().dtype(at::kByte));
+                const auto options = tensor(a[4]).options().dtype(at::kByte);
+                const at::Tensor ws = unlocked([&] { return at::empty({bytes}, options); });
                 Arg w;
                 w.fill(ws);
-                return g_entry.gemm_nt_ws(ta.get(), sfa.get(), tb.get(), sfb.get(), d.get(), nullptr, recipe, disable,
-                                          epilogue, &w.d, stream);
+                return call(g_entry.gemm_nt_ws, ta.get(), sfa.get(), tb.get(), sfb.get(), d.get(), nullptr, recipe,
+                            disable, epilogue, &w.d, stream);
             }
         }
-        return g_entry.gemm_nt(ta.get(), sfa.get(), tb.get(), sfb.get(), d.get(), c.get(), recipe, disable, epilogue, stream);
+        return call(g_entry.gemm_nt, ta.get(), sfa.get(), tb.get(), sfb.get(), d.get(), c.get(), recipe, disable,
+                    epilogue, stream);
     });
 }
 
@@ -174,10 +192,10 @@ PyObject* gemm_nt(PyObject*, PyObject* const* a, Py_ssize_t n) {
 PyObject* contiguous(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return guarded(n, 13, [&] {
         const Arg ta(a[0]), sfa(a[1]), tb(a[2]), sfb(a[3]), d(a[4]), layout(a[5]);
-        return g_entry.contiguous(ta.get(), sfa.get(), tb.get(), sfb.get(), d.get(), layout.get(),
-                                  pointer<const dg_recipe>(a[6]), (int32_t)integer(a[7]), (int32_t)integer(a[8]),
-                                  (int32_t)integer(a[9]), (int32_t)integer(a[10]), pointer<const dg_epilogue>(a[11]),
-                                  pointer<void>(a[12]));
+        return call(g_entry.contiguous, ta.get(), sfa.get(), tb.get(), sfb.get(), d.get(), layout.get(),
+                    pointer<const dg_recipe>(a[6]), (int32_t)integer(a[7]), (int32_t)integer(a[8]),
+                    (int32_t)integer(a[9]), (int32_t)integer(a[10]), pointer<const dg_epilogue>(a[11]),
+                    pointer<void>(a[12]));
     });
 }
 
@@ -185,9 +203,9 @@ PyObject* contiguous(PyObject*, PyObject* const* a, Py_ssize_t n) {
 PyObject* masked(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return guarded(n, 11, [&] {
         const Arg ta(a[0]), sfa(a[1]), tb(a[2]), sfb(a[3]), d(a[4]), masked_m(a[5]);
-        return g_entry.masked(ta.get(), sfa.get(), tb.get(), sfb.get(), d.get(), masked_m.get(), (int32_t)integer(a[6]),
-                              pointer<const dg_recipe>(a[7]), (int32_t)integer(a[8]), pointer<const dg_epilogue>(a[9]),
-                              pointer<void>(a[10]));
+        return call(g_entry.masked, ta.get(), sfa.get(), tb.get(), sfb.get(), d.get(), masked_m.get(),
+                    (int32_t)integer(a[6]), pointer<const dg_recipe>(a[7]), (int32_t)integer(a[8]),
+                    pointer<const dg_epilogue>(a[9]), pointer<void>(a[10]));
     });
 }
 
@@ -195,7 +213,8 @@ PyObject* masked(PyObject*, PyObject* const* a, Py_ssize_t n) {
 PyObject* cast(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return guarded(n, 6, [&] {
         const Arg x(a[0]), q(a[1]), sf(a[2]);
-        return g_entry.cast(x.get(), q.get(), sf.get(), (int32_t)integer(a[3]), (int32_t)integer(a[4]), pointer<void>(a[5]));
+        return call(g_entry.cast, x.get(), q.get(), sf.get(), (int32_t)integer(a[3]), (int32_t)integer(a[4]),
+                    pointer<void>(a[5]));
     });
 }
 
@@ -205,9 +224,9 @@ PyObject* dispatch(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return guarded(n, 14, [&] {
         const Arg x(a[0]), x_sf(a[1]), topk(a[2]), topk_w(a[3], true), out(a[7]), sf(a[8]), layout(a[9]), pos(a[10]),
             w(a[11], true), ws(a[12]);
-        return g_entry.dispatch(x.get(), x_sf.get(), topk.get(), topk_w.get(), (int32_t)integer(a[4]),
-                                (int32_t)integer(a[5]), (int32_t)integer(a[6]), out.get(), sf.get(), layout.get(),
-                                pos.get(), w.get(), ws.get(), pointer<void>(a[13]));
+        return call(g_entry.dispatch, x.get(), x_sf.get(), topk.get(), topk_w.get(), (int32_t)integer(a[4]),
+                    (int32_t)integer(a[5]), (int32_t)integer(a[6]), out.get(), sf.get(), layout.get(), pos.get(),
+                    w.get(), ws.get(), pointer<void>(a[13]));
     });
 }
 
@@ -215,8 +234,8 @@ PyObject* dispatch(PyObject*, PyObject* const* a, Py_ssize_t n) {
 PyObject* swiglu(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return guarded(n, 8, [&] {
         const Arg x(a[0]), w(a[1], true), layout(a[2], true), q(a[4]), sf(a[5]);
-        return g_entry.swiglu(x.get(), w.get(), layout.get(), real(a[3]), q.get(), sf.get(), (int32_t)integer(a[6]),
-                              pointer<void>(a[7]));
+        return call(g_entry.swiglu, x.get(), w.get(), layout.get(), real(a[3]), q.get(), sf.get(),
+                    (int32_t)integer(a[6]), pointer<void>(a[7]));
     });
 }
 
@@ -224,9 +243,9 @@ PyObject* swiglu(PyObject*, PyObject* const* a, Py_ssize_t n) {
 PyObject* contiguous_swiglu(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return guarded(n, 12, [&] {
         const Arg ta(a[0]), sfa(a[1]), tb(a[2]), sfb(a[3]), layout(a[4]), w(a[5], true), q(a[7]), sf(a[8]);
-        return g_entry.contiguous_swiglu(ta.get(), sfa.get(), tb.get(), sfb.get(), layout.get(), w.get(), real(a[6]),
-                                         q.get(), sf.get(), (int32_t)integer(a[9]), (int32_t)integer(a[10]),
-                                         pointer<void>(a[11]));
+        return call(g_entry.contiguous_swiglu, ta.get(), sfa.get(), tb.get(), sfb.get(), layout.get(), w.get(),
+                    real(a[6]), q.get(), sf.get(), (int32_t)integer(a[9]), (int32_t)integer(a[10]),
+                    pointer<void>(a[11]));
     });
 }
 
@@ -234,8 +253,8 @@ PyObject* contiguous_swiglu(PyObject*, PyObject* const* a, Py_ssize_t n) {
 PyObject* masked_swiglu(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return guarded(n, 11, [&] {
         const Arg ta(a[0]), sfa(a[1]), tb(a[2]), sfb(a[3]), masked_m(a[4]), w(a[6], true), q(a[8]), sf(a[9]);
-        return g_entry.masked_swiglu(ta.get(), sfa.get(), tb.get(), sfb.get(), masked_m.get(), (int32_t)integer(a[5]),
-                                     w.get(), real(a[7]), q.get(), sf.get(), pointer<void>(a[10]));
+        return call(g_entry.masked_swiglu, ta.get(), sfa.get(), tb.get(), sfb.get(), masked_m.get(),
+                    (int32_t)integer(a[5]), w.get(), real(a[7]), q.get(), sf.get(), pointer<void>(a[10]));
     });
 }
 
@@ -243,7 +262,7 @@ PyObject* masked_swiglu(PyObject*, PyObject* const* a, Py_ssize_t n) {
 PyObject* combine(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return guarded(n, 5, [&] {
         const Arg y(a[0]), pos(a[1]), w(a[2], true), out(a[3]);
-        return g_entry.combine(y.get(), pos.get(), w.get(), out.get(), pointer<void>(a[4]));
+        return call(g_entry.combine, y.get(), pos.get(), w.get(), out.get(), pointer<void>(a[4]));
     });
 }
 
