@@ -190,7 +190,7 @@ fp8_gemm_1d2d_pipe_kernel(const Fp8GemmArgs p_arg, const int num_m_blocks, const
     if constexpr (PERSIST) {
         if (lt != slot) __syncthreads();   // every wave is done with the previous tile's LDS
         if constexpr (TAB)
-            t = table_tile_coords<BN>(lt, p.m, s_tab, __builtin_amdgcn_readfirstlane(s_tab_n[0]),
+            t = table_tile_coords<BN>(lt, slot, p.m, s_tab, __builtin_amdgcn_readfirstlane(s_tab_n[0]),
                                       __builtin_amdgcn_readfirstlane(s_tab_n[1]), num_n_blocks, raster_gm);
         else
             t = decode_tile_persistent<BM, BN, KIND, NT>(lt, p.m, p.n, p.num_groups, p.layout, p.align_m, p.zero_padding,

@@ -312,12 +312,18 @@ __device__ __forceinline__ void build_block_table(const int32_t* __restrict__ la
     if (lane == 0) counts[0] = nf, counts[1] = nh;
 }
 
-// Tile lt of the launch's sequence from the block table; done past its end.
+// Tile of workgroup `slot` in the round that starts at lt - slot of the launch's
+// sequence, from the block table; done past its end. The last round runs backwards
+// over the workgroups: the ones that got the round before's last, 128-row tiles take
+// its tiles, instead of the ones that just had a 256-row tile (us, forwards ->
+// backwards, 16 experts: 2000 tokens, 4096 x 7168 178 -> 156 and 4096 x 2048 64 -> 58;
+// 8 experts, 3000 tokens, 4096 x 7168 171 -> 148).
 template <int BN>
-__device__ __forceinline__ PTile table_tile_coords(int lt, int m, const uint32_t* tab, int nf, int nh, int num_n_blocks,
-                                                   int raster_gm) {
+__device__ __forceinline__ PTile table_tile_coords(int lt, int slot, int m, const uint32_t* tab, int nf, int nh,
+                                                   int num_n_blocks, int raster_gm) {
     PTile t{};
-    const int fulls = nf * num_n_blocks;
+    const int fulls = nf * num_n_blocks, grid = gridDim.x;
+    if (lt - slot + grid >= fulls + nh * num_n_blocks) lt += grid - 1 - 2 * slot;
     const bool full = lt < fulls;
     if (lt >= fulls + nh * num_n_blocks) {
         t.done = 1;
