@@ -399,23 +399,24 @@ int64_t dense_split_columns(int64_t m_rows, int64_t n, int64_t k, int cus) {
     return best < 0.95 * whole ? best_n1 : 0;
 }
 
-// Row split of an m-grouped contiguous call (m_indices layout) whose 256 x 256 tiles
-// leave the last round nearly empty (35 M blocks x 16: 2 rounds and 48 tiles): rows
-// [0, r1) run as 256 x 256 tiles and rows [r1, M) as smaller ones. r1 is a multiple of
-// 256 and segments start on the M alignment, so each part is itself an m_indices
-// layout; every tile shape computes its outputs with the same arithmetic, so the
-// result is bitwise that of one launch. Returns r1 and the second launch's tile, or
-// 0 when the last round is more than 3/16 full, the per-round cost model gains less
-// than 11% or K is under 4096. Since the persistent walk cuts tiles from the segments'
-// own starts and leaves padding blocks out (its rounds no longer follow from M), one
-// launch is the faster one wherever the split was measured against it (8 experts, us,
-// split / one launch: 9216 x 4096 x 4096 205 / 183, 16768 x 4096 x 4096 321 / 308,
-// 33792 x 4096 x 7168 1013 / 982), so the split is bounded to the launches that it was
-// built for.
-int64_t contiguous_split_rows(int64_t m_rows, int64_t n, int64_t k, int cus, int align_m, TileConfig& hi_tile) {
-    if (k < 4096) return 0;
-    const int64_t left = ceil_div(m_rows, 256) * ceil_div(n, 256) % cus;
-    if (left == 0 || 16 * left > 3 * (int64_t)cus) return 0;
+// Row split of a persistent m-grouped contiguous call (m_indices layout) of one group
+// whose 256 x 256 tiles leave the last round partly empty: rows [0, r1) run as
+// 256 x 256 tiles and rows [r1, M) as smaller ones. r1 is a multiple of 256, so each
+// part is itself an m_indices layout; every tile shape computes its outputs with the
+// same arithmetic, so the result is bitwise that of one launch. Returns r1 and the
+// second launch's tile, or 0 when the per-round cost model gains less than 5% or K is
+// under 4096.
+// One group only: its rounds follow from M. Several segments with odd numbers of 128-row
+// blocks make more, shorter tiles, so that the first part overflows its rounds as well.
+// Measured (us, one launch -> split): one group, 4608 x 4096 x 4096 118 -> 100, x 7168
+// 192 -> 159, 5120 x 4096 x 7168 191 -> 167, 9216 x 4096 x 7168 302 -> 277,
+// 4864 x 7168 x 7168 288 -> 270, 16768 x 4096 x 4096 295 -> 301 (the smallest modelled
+// gain that splits, 5.8%: even); 8 groups, 4480 x 4096 x 4096 111 -> 127 and x 7168
+// 170 -> 179, 4 groups of 9 blocks 107 -> 115, 2 of 17 and 19 116 -> 124 (2 of 18 blocks,
+// all even: 120 -> 97, but half of the sizes with an even sum are not).
+int64_t contiguous_split_rows(int64_t m_rows, int64_t n, int64_t k, int64_t groups, int cus, int align_m,
+                              TileConfig& hi_tile) {
+    if (k < 4096 || groups != 1) return 0;
     struct Part { int bm, bn; double eff; };
     static const Part parts[] = {{256, 128, 1.00}, {128, 256, 0.97}, {128, 128, 0.80}};   // as in choose_tile_1d2d
     constexpr double t256 = 256.0 * 256 / 1.32;
@@ -433,7 +434,7 @@ int64_t contiguous_split_rows(int64_t m_rows, int64_t n, int64_t k, int cus, int
                                 rounds(ceil_div(rows2, p.bm) * ceil_div(n, p.bn)) * (p.bm * p.bn / p.eff);
             if (cost < best - 1e-9) best = cost, best_r1 = mb1 * 256, hi_tile = TileConfig{p.bm, p.bn, 2};
         }
-    return best < 0.89 * whole ? best_r1 : 0;
+    return best < 0.95 * whole ? best_r1 : 0;
 }
 
 // Whether a dense call on 256 x 256 tiles runs as persistent workgroups (variant 4):
@@ -766,7 +767,7 @@ void run_gemm(GemmKind kind, const Operands& o, const Recipe& r, int64_t m, int6
         }
         if (kind == kContiguous && tv == 0 && t.variant == 4) {
             TileConfig ht{};
-            const int64_t r1 = contiguous_split_rows(m_rows, n, k, args.grid_limit, align_m, ht);
+            const int64_t r1 = contiguous_split_rows(m_rows, n, k, groups, args.grid_limit, align_m, ht);
             if (r1 > 0) {
                 t_last_config += " split_m=" + std::to_string(r1) + ":" + std::to_string(ht.block_m) + "x" +
                                  std::to_string(ht.block_n);

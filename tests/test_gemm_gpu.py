@@ -378,16 +378,16 @@ def _contiguous_case(ms, aligned, n, k):
     assert torch.equal(d.view(torch.int16), first.view(torch.int16))
 
 
-@pytest.mark.parametrize('ms,mn_major', [(None, False), ([2000, 0, 4500, 2200], True)])
-def test_contiguous_row_split_equals_one_launch(ms, mn_major):
-    """m-grouped contiguous calls (K >= 4096; here fewer than four rounds of tiles)
-    whose 256 x 256 tiles would leave the last round mostly empty run as two
-    launches (the first rows on 256 x 256 tiles, the last M blocks on smaller
-    ones): bitwise the single 256 x 256 launch, padding rows untouched, and rows
-    on both sides of the split against the oracle. Cases: 8 experts with
-    Dirichlet sizes over 8192 tokens (35 M blocks, 2.2 rounds) and a split inside
-    a segment after an empty expert, with MN-major SFA. (At four rounds or more
-    the first part runs persistent, test_many_rounds_routes_persistent.)"""
+@pytest.mark.parametrize('ms,mn_major,two_launches', [(None, False, False), ([2000, 0, 4500, 2200], True, False),
+                                                      ([9000], True, True), ([9000], False, True)])
+def test_contiguous_row_split_equals_one_launch(ms, mn_major, two_launches):
+    """m-grouped contiguous calls (K >= 4096) whose 256 x 256 tiles would leave the last
+    round mostly empty: one group runs as two launches (the first rows on 256 x 256
+    tiles, the last M blocks on smaller ones), several groups as one. Bitwise the
+    single per-tile 256 x 256 launch, padding rows untouched, and rows around where
+    one group is split against the oracle. Cases: 8 experts with Dirichlet sizes over
+    8192 tokens (35 M blocks, 2.2 rounds), an empty expert and long segments, and one
+    expert of 9000 rows, with K- and MN-major SFA."""
     n, k = 4096, 4096
     if ms is None:
         ms, aligned = gen.contiguous_sizes(8, 8192, seed=7)
@@ -420,7 +420,8 @@ def test_contiguous_row_split_equals_one_launch(ms, mn_major):
 
     split, cfg = run()
     print(cfg, flush=True)
-    assert 'split_m=' in cfg, cfg
+    if deep_gemm.get_num_sms() >= 256:
+        assert ('split_m=' in cfg) == two_launches and ' v4 ' in cfg, cfg
     try:
         deep_gemm.set_tile_override(256, 256, variant=2)
         whole, cfg1 = run()
@@ -432,7 +433,7 @@ def test_contiguous_row_split_equals_one_launch(ms, mn_major):
     valid = torch.from_numpy(layout_np >= 0).to(DEV)
     assert bool((split.view(torch.int16)[~valid] == SENTINEL).all()), 'padding rows touched'
     # rows on both sides of the split row, and the first and last valid rows, against the oracle
-    r1 = int(cfg.split('split_m=')[1].split(':')[0])
+    r1 = int(cfg.split('split_m=')[1].split(':')[0]) if 'split_m=' in cfg else 8192
     cand = [0, r1 - 2, r1 - 1, r1, r1 + 1, int(np.nonzero(layout_np >= 0)[0][-1])]
     rows = np.array(sorted({r for r in cand if 0 <= r < m_pad and layout_np[r] >= 0}))
     a_deq = oquant.dequant_per_token(aq[rows].view(torch.uint8).cpu().numpy(), asf[rows].cpu().numpy())
@@ -1011,9 +1012,7 @@ def test_masked_routing_persistent_when_sparse(expected_m, persistent):
 def test_many_rounds_routes_persistent(case, k, persistent):
     """Contiguous calls, and dense calls with K <= 2048, with at least four rounds
     of 256 x 256 tiles on the CUs (BF16 D, no C) run the persistent walk by
-    default; the bits are those of the forced per-tile launch. The contiguous
-    K = 4096 call (66 M blocks: 4.1 rounds) also takes the row split, its first
-    64 M blocks persistent and the last rows on smaller tiles."""
+    default, in one launch; the bits are those of the forced per-tile launch."""
     print(f'many-rounds routing {case} k={k}', flush=True)
     if case == 'dense':
         m, n = 4096, 16384   # 16 x 64 = 1024 tiles: four rounds on 256 CUs
@@ -1043,7 +1042,7 @@ def test_many_rounds_routes_persistent(case, k, persistent):
     print(cfg, '|', cfg_ref, flush=True)
     if deep_gemm.get_num_sms() >= 256:
         assert ('v4' in cfg) == persistent
-        assert ('split_m=16384:' in cfg) == (case == 'contiguous' and k == 4096), cfg
+        assert 'split_m=' not in cfg, cfg
     assert torch.equal(ref.view(torch.int16), got.view(torch.int16))
 
 

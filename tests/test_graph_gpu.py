@@ -125,7 +125,7 @@ def test_graph_split_calls():
     replay_matches_eager(lambda: deep_gemm.fp8_gemm_nt(a, b, d), d)
     assert 'split_n=' in deep_gemm.get_last_config()
 
-    ms, aligned = gen.contiguous_sizes(8, 8192, seed=7)   # 8832 rows: 35 M blocks, 2.2 rounds
+    ms, aligned = [9000], [9088]   # one group: 36 M blocks, 2.25 rounds
     n, k = 4096, 4096
     m_pad = sum(aligned)
     layout_np = np.full(m_pad, -1, dtype=np.int32)
@@ -135,9 +135,9 @@ def test_graph_split_calls():
         start += ai
     layout = gen.to_dev(layout_np)
     ca = deep_gemm.per_token_cast_to_fp8(torch.randn((m_pad, k), generator=g, device=DEV).bfloat16(), use_ue8m0=False)
-    bq = torch.empty((8, n, k), dtype=torch.float8_e4m3fn, device=DEV)
-    bs = torch.empty((8, n // 128, k // 128), device=DEV)
-    for e in range(8):
+    bq = torch.empty((1, n, k), dtype=torch.float8_e4m3fn, device=DEV)
+    bs = torch.empty((1, n // 128, k // 128), device=DEV)
+    for e in range(1):
         bq[e], bs[e] = deep_gemm.per_block_cast_to_fp8(torch.randn((n, k), generator=g, device=DEV).bfloat16(),
                                                        use_ue8m0=False)
     dc = torch.empty((m_pad, n), dtype=torch.bfloat16, device=DEV)
