@@ -353,7 +353,7 @@ __device__ __forceinline__ void masked_pass(const Fp8GemmArgs& p, uint8_t* smem,
         __syncthreads();
         const SwigluOut o{p.sw_q, p.sw_ldq, p.sw_q_gs, p.sw_sf, p.sw_sf_sm, p.sw_sf_sk,
                           p.sw_sf_gs, p.sw_w, p.sw_w_gs, p.sw_clamp};
-        Buf::template run<NW>(smem, nullptr, wave, lane, r0, g, n0 >> 8, o, p.m - 1, [](int) { return 0; },
+        Buf::template run<NW>(smem, nullptr, wave, lane, r0, g, n0 >> 8, o, p.m - 1, ROWS, [](int) { return 0; },
                               [&](int m, int, bool& st, bool& z) {
                                   st = m < m_g;
                                   z = false;

@@ -774,9 +774,11 @@ fp8_gemm_1d2d_pipe_kernel(const Fp8GemmArgs p_arg, const int num_m_blocks, const
         __syncthreads();
         const int m_lo = npass == 2 ? m0 + pass * 128 : m0;
         const int m_hi = TAB ? t.row_end : npass == 2 ? m_lo + 128 : m0 + BM;
+        // (a 128-row tile of the table: half of the phase's steps)
+        const int tile_rows = TAB ? (a_rows + 3) & ~3 : BM;
         const SwigluOut o{p.sw_q, p.sw_ldq, p.sw_q_gs, p.sw_sf, p.sw_sf_sm, p.sw_sf_sk,
                           p.sw_sf_gs, p.sw_w, p.sw_w_gs, p.sw_clamp};
-        Buf::template run<NW>(smem, silu, wave, lane, m0, KIND == kMasked ? t.g : 0, n0 >> 8, o, p.m - 1,
+        Buf::template run<NW>(smem, silu, wave, lane, m0, KIND == kMasked ? t.g : 0, n0 >> 8, o, p.m - 1, tile_rows,
                               [&](int m) { return KIND == kContiguous ? p.layout[min(m, p.m - 1)] : 0; },
                               [&](int m, int id, bool& st, bool& z) {
                                   if constexpr (KIND == kContiguous) st = m < p.m && id >= 0, z = false;

@@ -251,10 +251,10 @@ struct SwigluTile {
     // fetch(row) loads what pred needs of a row (clamped to the rows that exist) and
     // is called, with the row's weight, one step ahead of its use: each was a
     // global round trip on every step's path. last_row: the last row of w. table: a
-    // filled SiluTable, or null.
+    // filled SiluTable, or null. rows: the tile's rows to visit, a multiple of 4.
     template <int NW, typename Fetch, typename Pred>
     __device__ static void run(const uint8_t* buf, const float* table, int wave, int lane, int row0, int g, int ib,
-                               const SwigluOut& o, int last_row, Fetch fetch, Pred pred) {
+                               const SwigluOut& o, int last_row, int rows, Fetch fetch, Pred pred) {
         static_assert(ROWS % (4 * NW) == 0, "whole row groups per wave");
         const int c16 = lane & 15;
         const int r_first = wave * 4 + (lane >> 4);
@@ -262,7 +262,7 @@ struct SwigluTile {
         int raw_next = fetch(row0 + r_first);
         float w_next = weight(row0 + r_first);
 #pragma unroll 1
-        for (int r = r_first; r < ROWS; r += 4 * NW) {
+        for (int r = r_first; r < rows; r += 4 * NW) {
             const int m = row0 + r;
             const uint4 gv = *reinterpret_cast<const uint4*>(buf + offset(r, 8 * c16));
             const uint4 uv = *reinterpret_cast<const uint4*>(buf + offset(r, 128 + 8 * c16));
