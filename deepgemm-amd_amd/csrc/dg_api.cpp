@@ -490,6 +490,12 @@ bool is_1d2d(const Operands& o, const Recipe& r) {
 
 // FP32 SF recipe of the reference's SM90 "1D1D" kernel (weight gradients):
 // A and B both 1 x 128 per row, both e4m3.
+// A persistent contiguous call in several launches (more blocks than its table holds).
+void record_table_launches(GemmKind kind, const TileConfig& t, const Fp8GemmArgs& args) {
+    const int launches = kind == kContiguous && t.variant == 4 ? fp8_table_launches(args) : 1;
+    if (launches > 1) t_last_config += " launches=" + std::to_string(launches);
+}
+
 bool is_1d1d(const Operands& o, const Recipe& r) {
     return o.a.dtype() == DG_E4M3 && o.b.dtype() == DG_E4M3 && o.sfa.dtype() == DG_F32 &&
            o.sfb.dtype() == DG_F32 && r.gran_mn_a == 1 && r.gran_k_a == 128 && r.gran_mn_b == 1 &&
@@ -773,6 +779,7 @@ void run_gemm(GemmKind kind, const Operands& o, const Recipe& r, int64_t m, int6
                                  std::to_string(ht.block_n);
                 Fp8GemmArgs lo = args;
                 lo.m = (int32_t)r1;
+                record_table_launches(kind, t, lo);
                 launch_fp8_gemm_1d2d_v2(kind, t, lo, stream);
                 // rows [r1, m): A rows, SFA rows (K- or MN-major: sfa_sm is the row
                 // stride), m_indices entries and D rows
@@ -788,6 +795,7 @@ void run_gemm(GemmKind kind, const Operands& o, const Recipe& r, int64_t m, int6
                 return;
             }
         }
+        record_table_launches(kind, t, args);
         if (t.variant == 8 || t.variant == 9)
             launch_fp8_gemm_tinym(args, t.variant == 8 ? 8 : 4, t.block_n, t.block_m, stream);
         else if (t.variant == 5)
@@ -1140,6 +1148,7 @@ void swiglu_l1_impl(GemmKind kind, const dg_tensor* a_, const dg_tensor* sfa_, c
     if (t.variant == 2 && !grouped_tile_ok(kind, 2, t.block_m, align_m))
         DG_UNSUPPORTED("M alignment for contiguous layout must be a multiple of 128 for the fused SwiGLU epilogue");
     record_config("fp8_gemm_1d2d_swiglu", kind, t, m, n, k, g);
+    record_table_launches(kind, t, args);
     if (t.variant == 5) {
         launch_fp8_gemm_masked_stream(args, 8, false, stream);
         return;

@@ -142,6 +142,11 @@ void launch_fp8_gemm_splitk(const Fp8GemmArgs& a, const SplitKPlan& plan, float*
 constexpr int kMaxTabBlocks = 3072;
 constexpr int kMaxTabBlocksEpi = 504;   // with the SwiGLU epilogue's table in LDS
 constexpr int kMaxTabGroups = 65535;
+// Launches of a persistent contiguous call.
+inline int fp8_table_launches(const Fp8GemmArgs& a) {
+    const int blocks = (a.m + 127) / 128, most = a.sw_q ? kMaxTabBlocksEpi : kMaxTabBlocks;
+    return a.num_groups > kMaxTabGroups ? 1 : (blocks + most - 1) / most;
+}
 
 // Launch the FP32-scale FP8 GEMM for `kind` with tile `cfg` on `stream`.
 // Throws dgm::Error on unsupported configurations or launch failures.

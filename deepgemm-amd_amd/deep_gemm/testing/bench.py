@@ -15,6 +15,8 @@ import os
 
 import torch
 
+from .. import _ffi
+
 __all__ = ['bench', 'bench_kineto', 'get_arch_major']
 
 _FLUSH_BYTES = 512 * 1024 * 1024
@@ -63,8 +65,8 @@ def bench_kineto(fn, kernel_names, num_tests: int = 30, suppress_kineto_output: 
     its symbol contains it. Returns a float for a string and a tuple for a tuple;
     a name no kernel matched gives 0. Unless `with_multiple_kernels`, a name that
     matches more than one distinct kernel is an error (as in the reference), except
-    for one library call that runs as two launches (a column or row split): then
-    each of its kernels ran once per call and the result is the call's time.
+    for one library call that runs as several launches (a column or row split, or the
+    parts of a long contiguous layout): then the result is the call's time.
     `fn` runs once untraced, then `num_tests` times in the traced window, each
     after a cache flush (`flush_l2`) and a call of `barrier` when given.
     `suppress_kineto_output` is accepted for signature compatibility.
@@ -78,6 +80,8 @@ def bench_kineto(fn, kernel_names, num_tests: int = 30, suppress_kineto_output: 
     cache = _flush_buffer() if flush_l2 else None
     fn()
     torch.cuda.synchronize()
+    config = _ffi.last_config()
+    parts = int(config.split(' launches=')[1].split()[0]) if ' launches=' in config else 1
     schedule = torch.profiler.schedule(wait=0, warmup=1, active=1, repeat=1)
     prof = torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA], schedule=schedule)
     with prof:
@@ -106,6 +110,10 @@ def bench_kineto(fn, kernel_names, num_tests: int = 30, suppress_kineto_output: 
                 times.append(sum(_device_time_us(e) / e.count for e in hits) / 1e6)
                 continue
             raise AssertionError(f'kernel name {name!r} matches several kernels: {[e.key for e in hits]}')
+        if not with_multiple_kernels and parts > 1 and len(hits) == 1 and 'dgm::' in hits[0].key and \
+                hits[0].count == parts * num_tests:
+            times.append(_device_time_us(hits[0]) / num_tests / 1e6)   # (one symbol, a launch per part)
+            continue
         total_us = sum(_device_time_us(e) for e in hits)
         count = sum(e.count for e in hits)
         times.append(total_us / count / 1e6 if count else 0.0)

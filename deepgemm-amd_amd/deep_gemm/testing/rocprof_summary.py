@@ -92,14 +92,15 @@ def mfma_utilization(busy_cycles: float, gui_cycles: float, kernel_us: float, si
 
 def dispatches_per_call(config: str) -> int:
     """Kernels one bench launch dispatches: a dense column split, a contiguous row
-    split or the split-K kernel (partials, then the reduction) runs two; a MoE
-    dispatch runs its count, scan, (segment starts,) scatter kernels; a launch of
+    split or the split-K kernel (partials, then the reduction) runs two; a contiguous
+    layout longer than a block table runs `launches`; a MoE dispatch runs its count, scan, (segment starts,) scatter kernels; a launch of
     several library calls (configs joined by ' + ') sums them."""
     if ' + ' in config:
         return sum(dispatches_per_call(c) for c in config.split(' + '))
     if config.startswith('moe_dispatch'):   # count, scan, (starts,) scatter
         return 3 if 'layout=masked' in config else 4
-    return 2 if ('split_n=' in config or 'split_m=' in config or ' splits=' in config) else 1
+    two = 'split_n=' in config or 'split_m=' in config or ' splits=' in config
+    return (int(config.split(' launches=')[1].split()[0]) if ' launches=' in config else 1) + int(two)
 
 
 def _workgroups(row) -> int:

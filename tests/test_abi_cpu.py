@@ -412,3 +412,18 @@ def test_ue8m0_row_groups_fit_the_grid(m, kernel):
                       fake((m, n), _ffi.DG_BF16), recipe=_ffi.recipe_struct(None, (1, 128), (1, 128)))
     assert st == _ffi.DG_ERR_HIP, msg   # (only for want of a device)
     assert f'ue8m0_{kernel} ' in deep_gemm.get_last_config()
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason='the accepted call would launch on fake addresses')
+@pytest.mark.parametrize('rows,launches', [(504 * 128, 1), (504 * 128 + 1, 2), (65536, 2), (1009 * 128, 3)])
+def test_fused_contiguous_launches_are_recorded(rows, launches):
+    """A layout of more 128-row blocks than the block table holds names its launches."""
+    g, inter, k = 2, 256, 1024
+    st = _ffi.lib.dg_m_grouped_fp8_gemm_nt_contiguous_swiglu(
+        *(ctypes.byref(x) for x in (
+            fake((rows, k), _ffi.DG_E4M3), fake((rows, k // 128), _ffi.DG_F32), fake((g, 2 * inter, k), _ffi.DG_E4M3),
+            fake((g, 2 * inter // 128, k // 128), _ffi.DG_F32), fake((rows,), _ffi.DG_I32))), None, 0.0,
+        ctypes.byref(fake((rows, inter), _ffi.DG_E4M3)), ctypes.byref(fake((rows, inter // 128), _ffi.DG_F32)), 0, 0, None)
+    assert st == _ffi.DG_ERR_HIP, _ffi.lib.dg_last_error()   # (only for want of a device)
+    cfg = deep_gemm.get_last_config()
+    assert ' v4 ' in cfg and (f' launches={launches}' in cfg if launches > 1 else 'launches' not in cfg), cfg

@@ -82,6 +82,8 @@ def test_dispatches_per_call():
     assert rs.dispatches_per_call('fp8_gemm_1d2d v2 kind=normal block_m=256 block_n=256 split_n=4096:256x192') == 2
     assert rs.dispatches_per_call('fp8_gemm_1d2d v2 kind=m_grouped_contiguous block_m=256 block_n=256 '
                                   'split_m=32768:128x128') == 2
+    assert rs.dispatches_per_call('fp8_gemm_1d2d v4 kind=m_grouped_contiguous block_m=256 block_n=256 m=1048576 n=256 '
+                                  'k=128 groups=2 launches=3') == 3
 
 
 def test_dispatches_per_call_split_k_and_joined_calls():

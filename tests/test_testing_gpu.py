@@ -67,3 +67,23 @@ def test_bench_kineto_split_call_is_one_call():
           f'whole call {t_call * 1e6:.1f} us', flush=True)
     assert 1.6 * t_avg < t < 2.4 * t_avg
     assert 0.5 * t_call < t <= 1.2 * t_call
+
+
+def test_bench_kineto_long_contiguous_layout_is_one_call():
+    """A contiguous layout of more blocks than one launch's table holds runs one kernel in
+    several launches: timed as one call, twice the per-launch average."""
+    rows, n, k = 128 * 3200, 256, 128
+    g = torch.Generator(device=DEV).manual_seed(6)
+    a = deep_gemm.per_token_cast_to_fp8(torch.randn((rows, k), generator=g, device=DEV).bfloat16(), use_ue8m0=False)
+    q, sf = deep_gemm.per_block_cast_to_fp8(torch.randn((n, k), generator=g, device=DEV).bfloat16(), use_ue8m0=False)
+    d = torch.empty((rows, n), dtype=torch.bfloat16, device=DEV)
+    idx = torch.zeros(rows, dtype=torch.int32, device=DEV)
+
+    def call():
+        deep_gemm.m_grouped_fp8_gemm_nt_contiguous(a, (q[None], sf[None]), d, idx)
+    call()
+    assert ' launches=2' in deep_gemm.get_last_config()
+    t = bench_kineto(call, 'gemm_', num_tests=10)
+    t_avg = bench_kineto(call, 'gemm_', num_tests=10, with_multiple_kernels=True)
+    print(f'long layout: bench_kineto {t * 1e6:.1f} us, per launch {t_avg * 1e6:.1f} us', flush=True)
+    assert 1.6 * t_avg < t < 2.4 * t_avg
