@@ -542,26 +542,32 @@ void launch_1d1d(bool k_grouped, const Fp8GemmArgs& args, hipStream_t stream, in
     launch_fp8_gemm_1d1d_pipe(k_grouped, t, args, stream);
 }
 
-// Workgroup shape of the UE8M0 tiny-M kernel for a dense call, or {256, 256, 2} where
-// the pipelined kernel is faster. Time per round of workgroups on the CUs, measured (us,
-// kb = K blocks; A e4m3, B e2m1): 32 x 32 4.5 + 0.115 kb, 32 x 64 6.5 + 0.19 kb, 64 x 32
-// 4 + 0.285 kb, 64 x 64 4.5 + 0.345 kb, pipelined 256 x 256 6 + 1.15 kb. Measured,
-// pipelined -> the chosen shape: 1 x 7168 x 7168 70 -> 8.6, 48 x 7168 x 7168 70 -> 17,
-// 200 x 7168 x 7168 72 -> 48, 400 x 2112 x 7168 74 -> 26, 48 x 24576 x 1536 21 -> 16,
-// 200 x 7168 x 2048 26 -> 16; it stays pipelined at 100 x 24576 x 1536 (21, 64 x 64 23)
-// and 400 x 7168 x 7168 (73, 79).
-TileConfig choose_ue8m0_tinym(int64_t m, int64_t n, int64_t k, int cus) {
+// Workgroup shape of the UE8M0 tiny-M kernel for a dense call (A e4m3), or {256, 256, 2}
+// where the pipelined kernel is faster. t0 + tk * K blocks: time per round of
+// workgroups on the CUs, measured (us). Measured, pipelined -> the chosen shape (weights
+// from HBM; B e2m1, in brackets e4m3): 1 x 7168 x 7168 71 -> 10.2 (82 -> 14), 64 x 7168 x
+// 7168 71 -> 20 (83 -> 31), 200 x 7168 x 7168 79 -> 51 (92 -> 65), 400 x 2112 x 7168 76 ->
+// 27 (99 -> 34), 64 x 24576 x 1536 22 -> 19 (24.5 -> 22), 200 x 7168 x 2048 26 -> 17 (30 ->
+// 21), 1600 x 576 x 7168 85 -> 28 (99 -> 34), 1 x 4096 x 1024 15.5 -> 5.7 (17 -> 7.4),
+// 200 x 4096 x 1024 17 -> 9.3 (18 -> 11), 64 x 7168 x 512 11.4 -> 6.5 (11.5 -> 7.1); it
+// stays pipelined at 100 x 24576 x 1536 (22, 64 x 64 23), 400 x 7168 x 7168 (82, 82),
+// 400 x 7168 x 512 (13, 18) and, B e4m3, 400 x 4096 x 1024 (18.4, 64 x 64 20; e2m1 goes
+// 17.5 -> 16.6). Over 272 sizes (1 to 1600 rows, N 256 to 32768, K 512 to 16384, either B)
+// no call is slower than pipelined; the shape chosen misses the best one by 19% at most
+// (100 x 2112 x 7168, e4m3: 28, 32 x 32 24).
+// The sums are grouped by wave, so a call's bits follow the kernel that its size picks.
+TileConfig choose_ue8m0_tinym(int64_t m, int64_t n, int64_t k, bool b_fp4, int cus) {
     struct Shape { int rows, cols; double t0, tk; };
-    static const Shape shapes[] = {{32, 32, 4.5, 0.115}, {32, 64, 6.5, 0.19}, {64, 32, 4.0, 0.285}, {64, 64, 4.5, 0.345}};
+    static const Shape e2m1[] = {{256, 256, 6.0, 1.15}, {32, 32, 4.5, 0.115}, {32, 64, 6.5, 0.19}, {64, 32, 4.0, 0.285},
+                                 {64, 64, 4.5, 0.345}};
+    static const Shape e4m3[] = {{256, 256, 6.8, 1.36}, {32, 32, 5.0, 0.25}, {32, 64, 6.8, 0.41}, {64, 32, 4.8, 0.45},
+                                 {64, 64, 5.5, 0.50}};
     const double kb = (double)k / 128;
-    // Up to 8 K blocks (pipelined at most 15 us, 6 here) a call keeps the sums in one
-    // chain: the bits of the same call with FP32 scales, which callers compare.
-    if (kb <= 8) return TileConfig{256, 256, 2};
-    double best = (double)ceil_div(ceil_div(m, 256) * ceil_div(n, 256), cus) * (6.0 + 1.15 * kb);
+    double best = 1e300;
     TileConfig out{256, 256, 2};
-    for (const auto& s : shapes) {
+    for (const auto& s : b_fp4 ? e2m1 : e4m3) {
         const double cost = (double)ceil_div(ceil_div(m, s.rows) * ceil_div(n, s.cols), cus) * (s.t0 + s.tk * kb);
-        if (cost < best) best = cost, out = TileConfig{s.rows, s.cols, 11};
+        if (cost < best) best = cost, out = TileConfig{s.rows, s.cols, s.rows == 256 ? 2 : 11};
     }
     return out;
 }
@@ -855,7 +861,7 @@ void run_gemm(GemmKind kind, const Operands& o, const Recipe& r, int64_t m, int6
         if (kind == kNormal && (tv == 0 || tv == 11) && fp8_fp4_tinym_supported(args)) {
             int cus = 256;
             try { cus = num_sms_now(); } catch (const Error&) {}
-            TileConfig t = choose_ue8m0_tinym(m, n, k, std::max(1, cus));
+            TileConfig t = choose_ue8m0_tinym(m, n, k, args.b_fp4 != 0, std::max(1, cus));
             if (tv == 11) t = {g_tile_m.load(), g_tile_n.load(), 11};
             if (t.variant == 11) {
                 record_config("fp8_fp4_gemm_ue8m0_tinym", kind, t, m, n, k, groups);

@@ -408,8 +408,8 @@ def test_ue8m0_row_groups_fit_the_grid(m, kernel):
     grid holds, the pipelined one beyond (never refused for the grid)."""
     n, k = 32, 32768
     st, msg = call_nt(fake((m, k), _ffi.DG_E4M3), fake((m, k // 512), _ffi.DG_I32, strides=(1, (m + 3) // 4 * 4)),
-                      fake((n, k), _ffi.DG_E4M3, addr=0x20000000), fake((n, k // 512), _ffi.DG_I32, strides=(1, n)),
-                      fake((m, n), _ffi.DG_BF16), recipe=_ffi.recipe_struct(None, (1, 128), (1, 128)))
+                      fake((n, k // 2), _ffi.DG_I8, addr=0x20000000), fake((n, k // 128), _ffi.DG_I32, strides=(1, n)),
+                      fake((m, n), _ffi.DG_BF16), recipe=_ffi.recipe_struct(None, (1, 128), (1, 32)))
     assert st == _ffi.DG_ERR_HIP, msg   # (only for want of a device)
     assert f'ue8m0_{kernel} ' in deep_gemm.get_last_config()
 

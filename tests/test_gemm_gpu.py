@@ -1229,12 +1229,44 @@ def test_ue8m0_pipe_dense(m, n, k, a_fp4, b_fp4, gka, gkb):
     outside = torch.ones_like(new, dtype=torch.bool)
     outside[:m, :n] = False
     assert bool((new.view(torch.int16)[outside] == SENTINEL).all())
-    # determinism (heuristic dispatch picks the pipelined kernel)
+    # determinism (few rows are the tiny-M kernel's by default, test_ue8m0_tiny_m)
     d = big[:m, :n]
-    for _ in range(20):
-        deep_gemm.fp8_fp4_gemm_nt(a, b, d, recipe_a=(1, gka), recipe_b=(1, gkb))
+    deep_gemm.set_tile_override(256, 256, variant=2)
+    try:
+        for _ in range(20):
+            deep_gemm.fp8_fp4_gemm_nt(a, b, d, recipe_a=(1, gka), recipe_b=(1, gkb))
+    finally:
+        deep_gemm.set_tile_override(0, 0)
     assert 'pipe' in deep_gemm.get_last_config()
     assert torch.equal(big.view(torch.int16), new.view(torch.int16))
+
+
+@pytest.mark.parametrize('m,n,k,b_fp4,kernel', [
+    (1, 64, 128, True, 'tinym'), (64, 4096, 512, True, 'tinym'), (100, 4096, 1024, False, 'tinym'),
+    (64, 520, 1152, True, 'tinym'), (400, 7168, 512, True, 'pipe'), (4096, 4096, 1024, False, 'pipe')])
+def test_ue8m0_few_rows_route(m, n, k, b_fp4, kernel):
+    """The kernel of a dense call follows from its size at every K; what it gives is the
+    pipelined kernel's result but for the order of the sums."""
+    g = torch.Generator(device=DEV).manual_seed(m + n + k)
+    x, w = torch.randn((m, k), generator=g, device=DEV).bfloat16(), torch.randn((n, k), generator=g, device=DEV).bfloat16()
+    pack = deep_gemm.get_mn_major_tma_aligned_packed_ue8m0_tensor
+    qa, sfa = deep_gemm.per_token_cast_to_fp8(x, use_ue8m0=True)
+    qb, sfb = (deep_gemm.per_token_cast_to_fp4(w, use_ue8m0=True, gran_k=32) if b_fp4 else
+               deep_gemm.per_token_cast_to_fp8(w, use_ue8m0=True))
+    a, b, outs = (qa, pack(sfa)), (qb, pack(sfb)), []
+    for v in (0, 2):
+        d = torch.empty((m, n), dtype=torch.bfloat16, device=DEV)
+        deep_gemm.set_tile_override(256 if v else 0, 256 if v else 0, variant=v)
+        try:
+            deep_gemm.fp8_fp4_gemm_nt(a, b, d, recipe_a=(1, 128), recipe_b=(1, 32 if b_fp4 else 128))
+            if v == 0 and deep_gemm.get_num_sms() >= 256:
+                assert f'ue8m0_{kernel} ' in deep_gemm.get_last_config()
+        finally:
+            deep_gemm.set_tile_override(0, 0)
+        outs.append(d.float())
+    torch.cuda.synchronize()
+    # (one BF16 rounding apart where FP32 sums of another order straddle one)
+    assert bool(((outs[0] - outs[1]).abs() <= outs[1].abs() * 2.0 ** -7 + 2.0 ** -15 * k ** 0.5 * 8).all())
 
 
 @pytest.mark.parametrize('out_f32,with_c', [(True, True), (True, False), (False, True)])
