@@ -322,13 +322,12 @@ TileConfig choose_tile_1d2d(GemmKind kind, int64_t m_rows, int64_t n, int64_t k,
     const int tv = g_tile_variant.load(), tm = g_tile_m.load(), tn = g_tile_n.load();
     // The pipelined kernel keeps one SFB value per K block in LDS (up to 1024 blocks).
     const bool pipe_ok = offsets_fit && ceil_div(k, 128) <= 1024;
-    // K % 128 != 0: the 256 x 256 pipelined tile is built for dense launches only,
-    // and an override takes it with whole K blocks only (the other tiles give the
-    // same bits).
-    const bool tile256_ok = k % 128 == 0;
+    // K % 128 != 0: the 256 x 256 pipelined tile is built for dense launches of one
+    // workgroup per tile only (the other tiles give the same bits).
+    const bool tile256_ok = k % 128 == 0 || kind == kNormal;
     if (tv == 4) {   // persistent form of the pipelined kernel
         if (!pipe_ok || tm != 256 || tn != 256) DG_UNSUPPORTED("tile override: the persistent kernel is 256 x 256");
-        if (!tile256_ok) DG_UNSUPPORTED("tile override: the 256 x 256 pipelined tile needs K % 128 == 0");
+        if (k % 128 != 0) DG_UNSUPPORTED("tile override: the persistent 256 x 256 tile needs K % 128 == 0");
         if (!grouped_tile_ok(kind, tv, tm, align_m)) DG_UNSUPPORTED("tile override block_m does not fit the M alignment");
         return {256, 256, 4};
     }
@@ -336,7 +335,7 @@ TileConfig choose_tile_1d2d(GemmKind kind, int64_t m_rows, int64_t n, int64_t k,
         const bool ok = tv == 1 ? fp8_1d2d_tile_supported(tm, tn) : (pipe_ok && fp8_1d2d_v2_tile_supported(tm, tn));
         if (!ok) DG_UNSUPPORTED("tile override not compiled");
         if (tv == 2 && tm == 256 && tn == 256 && !tile256_ok)
-            DG_UNSUPPORTED("tile override: the 256 x 256 pipelined tile needs K % 128 == 0");
+            DG_UNSUPPORTED("tile override: the 256 x 256 pipelined tile of grouped calls needs K % 128 == 0");
         if (!grouped_tile_ok(kind, tv, tm, align_m))
             DG_UNSUPPORTED("tile override block_m does not fit the M alignment");
         return {tm, tn, tv};
@@ -358,7 +357,7 @@ TileConfig choose_tile_1d2d(GemmKind kind, int64_t m_rows, int64_t n, int64_t k,
         if (whole_k_contiguous && c.bm == 256) continue;
         if (!grouped_tile_ok(kind, c.variant, c.bm, align_m)) continue;
         if (c.variant == 2 && !pipe_ok) continue;
-        if (c.variant == 2 && c.bm == 256 && c.bn == 256 && !tile256_ok && kind != kNormal) continue;
+        if (c.variant == 2 && c.bm == 256 && c.bn == 256 && !tile256_ok) continue;
         const int64_t tiles = ceil_div(m_rows, c.bm) * ceil_div(n, c.bn) * groups;
         const int64_t slots = (int64_t)cus * c.per_cu;
         const double rounds = (double)ceil_div(tiles, slots);

@@ -250,19 +250,38 @@ def test_grouped_validation():
 
 
 def test_k_tail_rejects_256x256_override():
-    """The 256 x 256 pipelined tile has no K-tail schedule (it would spill
-    registers): a tile override that would launch it with K % 128 != 0 (plain
-    or persistent) is refused on the host, before any launch."""
+    """The persistent 256 x 256 tile has no K-tail schedule, and the per-tile one has it for
+    dense calls only: a tile override that would launch another with K % 128 != 0 is
+    refused on the host, before any launch."""
     a, sfa, b, sfb, d = good_dense(512, 512, 1040)
     sfa = fake((512, 9), _ffi.DG_F32)
     sfb = fake((4, 9), _ffi.DG_F32)
-    for variant in (2, 4):
+    b3, sfb3, d3 = fake((1, 512, 1040), _ffi.DG_E4M3), fake((1, 4, 9), _ffi.DG_F32), fake((512, 512), _ffi.DG_BF16)
+    for variant, grouped in ((4, False), (2, True), (4, True)):
         deep_gemm.set_tile_override(256, 256, variant=variant)
         try:
-            st, msg = call_nt(a, sfa, b, sfb, d)
+            if grouped:
+                st = _ffi.lib.dg_m_grouped_fp8_fp4_gemm_nt_contiguous(
+                    *(ctypes.byref(x) for x in (a, sfa, b3, sfb3, d3, fake((512,), _ffi.DG_I32))), None, 0, 0, 0, -1,
+                    None, None)
+                msg = _ffi.lib.dg_last_error().decode()
+            else:
+                st, msg = call_nt(a, sfa, b, sfb, d)
         finally:
             deep_gemm.set_tile_override(0, 0)
-        assert st == _ffi.DG_ERR_UNSUPPORTED and 'K % 128 == 0' in msg, (variant, msg)
+        assert st == _ffi.DG_ERR_UNSUPPORTED and 'K % 128 == 0' in msg, (variant, grouped, msg)
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason='the accepted call would launch on fake addresses')
+def test_k_tail_takes_256x256_override():
+    """... and the dense per-tile one, which the heuristic takes too, is accepted."""
+    a, _, b, _, d = good_dense(512, 512, 1040)
+    deep_gemm.set_tile_override(256, 256, variant=2)
+    try:
+        st, msg = call_nt(a, fake((512, 9), _ffi.DG_F32), b, fake((4, 9), _ffi.DG_F32), d)
+    finally:
+        deep_gemm.set_tile_override(0, 0)
+    assert st == _ffi.DG_ERR_HIP and ' v2 kind=normal block_m=256 block_n=256 ' in deep_gemm.get_last_config(), msg
 
 
 def test_fused_swiglu_host_checks():
@@ -301,7 +320,7 @@ def test_fused_swiglu_host_checks():
     assert st == _ffi.DG_ERR_INVALID and 'gl.size(0) ==' in msg
     st, msg = contiguous(a=fake((m, k), _ffi.DG_E4M3, device=-1))
     assert st == _ffi.DG_ERR_INVALID and 'on_device' in msg
-    # 256 x 256 tiles need K % 128 == 0 (the K-tail 256-row schedule is not built)
+    # 256 x 256 tiles need K % 128 == 0 (their K-tail schedule is built for dense calls)
     a_t, sfa_t = fake((m, 1040), _ffi.DG_E4M3), fake((m, 9), _ffi.DG_F32)
     b_t, sfb_t = fake((g, n, 1040), _ffi.DG_E4M3), fake((g, n // 128, 9), _ffi.DG_F32)
     deep_gemm.set_tile_override(256, 256, variant=2)
