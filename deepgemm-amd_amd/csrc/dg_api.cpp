@@ -49,8 +49,8 @@ constexpr int64_t kTinyMWideMaxTiles = 64;   // 128 x 128 tiles of the tiled lau
 constexpr int kTinyMStreamGrid = 64;
 // Dense calls whose tiles come out as 128 x 128 take the kernel that splits K blocks over
 // two wave groups up to three quarters of a round of tiles, with K from 2048 and B of at
-// most 32 MB: 19-25% faster there with the weights in cache (the figures are beside the
-// kernel), even to 6% with weights from HBM. Beyond, HBM latency shows, as it keeps fewer stages
+// most 32 MB: 18-24% less time there with the weights in cache (the figures are beside the
+// kernel), 1-8% with weights from HBM. Beyond, HBM latency shows, as it keeps fewer stages
 // in flight (weights from HBM, pipelined -> split): 1024 x 4096 x 7168 (a full round)
 // 42.4 -> 44.1 us, 256 x 7168 x 7168 (51 MB) 41.5 -> 44.7; K = 1536 and less is even or
 // gains under 1 us; a partial last K block lost 5% (2000 x 1536 x 3008), so it has no
@@ -453,8 +453,11 @@ bool is_persistent_route(GemmKind kind, const TileConfig& t, const Fp8GemmArgs& 
 // other tile (us, 128 x 256 -> persistent): 4 experts 1536 x 4096 x 7168 (192 tiles)
 // 81 -> 110; 2560 x 4096 x 4096 (320) 76 -> 63, 2048 x 7168 x 2048 (448) 49 -> 45,
 // 5120 x 4096 x 4096 136 -> 120, 32 experts 12288 x 4096 x 7168 502 -> 380, 36864 x
-// 7168 x 2048 766 -> 589; slower only where every segment is one block (16 experts
-// 4096 x 4096 x 2048 53 -> 63, but 32 experts 5120 x 4096 x 2048 80 -> 66). One
+// 7168 x 2048 766 -> 589. Slower by up to 15% where most segments are one block and the
+// 128 x 256 tiles make just two rounds (16 experts, 24 blocks of rows in 32, 4096 x 4096 x
+// 2048 55 -> 58; 8 experts, 13 blocks in 16, 2048 x 7168 x 2048 51 -> 58); M and the
+// groups do not tell those from calls that gain as much (16 experts of two blocks each, the
+// same sizes, 59 -> 50), since how many blocks hold rows is in m_indices. One
 // workgroup per 256-row tile at multiples of 256 rows took 515 and 606 us on the two
 // 32-expert calls.
 bool is_table_route(int64_t m_rows, int64_t n, int64_t k, int64_t groups, int cus, int align_m) {

@@ -16,9 +16,10 @@
 // differently from the single-chain kernels, so the bits differ: a configuration of its
 // own (variant 12).
 //
-// What bounds it: weights in cache, the LDS (192 KB through it per pair of blocks, 0.64 us
-// of the 1.07 that a pair takes) and the one barrier of a pair; weights from HBM, the
-// latency of a pair's loads with two pairs of stages in 160 KB. Measured (us, the
+// What bounds it: the chain of a pair of blocks, its one barrier and the latency of the
+// loads that it waits for, with two pairs of stages in 160 KB: at 517 x 4096 x 7168 a busy
+// CU's LDS reads take 29% of its cycles, its MFMAs 40% (21% and 30% with weights
+// from HBM, where those loads take longer). Measured (us, the
 // pipelined kernel's 128 x 128 tiles -> this): 517 x 4096 x 7168 40.5 -> 32.0,
 // 300 x 2112 x 7168 40.8 -> 31.7, 700 x 4096 x 4096 25.6 -> 20.7, 400 x 4096 x 2048
 // 15.3 -> 12.6, 140 x 1536 x 16384 84 -> 64; with weights from HBM 47.3 -> 46.9 (640 rows),

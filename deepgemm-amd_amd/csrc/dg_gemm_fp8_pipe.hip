@@ -553,8 +553,8 @@ fp8_gemm_1d2d_pipe_kernel(const Fp8GemmArgs p_arg, const int num_m_blocks, const
     // Measured, interleaved runs: config-2 step 870-878 against 873-888 us,
     // contiguous 1633-1639 against 1649-1657 us (with warm caches in a stripped
     // copy, 2-3% per shape); with masks that stop everything (0) it was 1-3%
-    // slower than the compiler's order. 1D1D tiles keep the compiler's order
-    // (pinned, the K-grouped launch took 2117-2139 against 2073-2113 us).
+    // slower than the compiler's order. The 256 x 256 1D1D tile keeps the compiler's order
+    // (pinned, the K-grouped launch was 0.8% slower); the 128 x 128 one is pinned.
     // Persistent tiles take it (config-2 shapes all as persistent launches: 945
     // against 980 us; sparse masked groups 1-2% faster).
     constexpr bool PIN_PROMO = !SB1D || NW == 4;

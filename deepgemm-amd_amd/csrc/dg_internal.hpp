@@ -162,7 +162,7 @@ void launch_fp8_gemm_1d2d_v2(GemmKind kind, const TileConfig& cfg, const Fp8Gemm
 bool fp8_1d2d_v2_tile_supported(int block_m, int block_n);
 
 // Dense calls of at most a round of 128 x 128 tiles, even and odd K blocks on two
-// groups of waves (dg_gemm_fp8_ksplit.hip): BF16 D without C, K a multiple of 16.
+// groups of waves (dg_gemm_fp8_ksplit.hip): BF16 D without C, K a multiple of 128.
 bool fp8_ksplit_supported(const Fp8GemmArgs& args);
 void launch_fp8_gemm_ksplit(const Fp8GemmArgs& args, hipStream_t stream);
 

@@ -227,7 +227,7 @@ def summarize(args):
                  f'bench.py (after a cache flush, {rot} back-to-back launches of one shape on rotating buffer '
                  'sets, repeated), next to the HIP-event average per launch that bench.py measured in the '
                  'same run.\n')
-    lines.append('Commands (repository root on the GPU box; `OUT` = an output folder):\n')
+    lines.append('Commands (repository root; `OUT` = an output folder):\n')
     lines.append('```')
     for c in args.command or []:
         lines.append(c)
